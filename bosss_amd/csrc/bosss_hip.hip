@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/bosss_hip.h"
+#include "assemble_linear.hpp"
 #include "devbuf.hpp"
 #include "dg_kernels.hpp"
 #include "registry.hpp"
@@ -85,6 +86,9 @@ struct bosss_op {
   int ncolors;
   int32_t *d_color, *d_cols;
   std::vector<int32_t> cols_host;
+  // direct assembly of the linear forms: reference matrices (made at creation), per-cell coefficients
+  bool merged_slots = false;   // a row holds one neighbour across several faces (or itself)
+  double *d_lintab = nullptr, *d_lincoef = nullptr;
   // tile shape of the block-ELL apply (panel size NL): tuned on the first device apply
   bool spmv_tuned = false;
   int spmv_nl = 0;
@@ -433,7 +437,12 @@ int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tabl
       if (rc) { (void)hipFree(op->tables); delete op; return rc; }
     }
   }
-  if ((rc = ks->prepare()) != 0) { (void)hipFree(op->tables); delete op; return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc); }
+  if (kind == BOSSS_FORM_SIP || kind == BOSSS_FORM_ADVDIFF) {
+    std::vector<double> T;
+    linear_reference_matrices(t->D, t->N, t->Kv, t->Ke, grid->pair, t->vol_weights, t->phi, t->dphi, t->face_weights, t->trace, t->dtrace, T);
+    if ((rc = upload(&op->d_lintab, T.data(), T.size()))) { bosss_hip_op_destroy(op); return rc; }
+  }
+  if ((rc = ks->prepare()) != 0) { bosss_hip_op_destroy(op); return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc); }
   *out = op;
   return BOSSS_OK;
 }
@@ -449,6 +458,8 @@ int bosss_hip_op_destroy(bosss_op* op) {
   if (op->d_color) (void)hipFree(op->d_color);
   if (op->d_cols) (void)hipFree(op->d_cols);
   if (op->d_first) (void)hipFree(op->d_first);
+  if (op->d_lintab) (void)hipFree(op->d_lintab);
+  if (op->d_lincoef) (void)hipFree(op->d_lincoef);
   delete op;
   return BOSSS_OK;
 }
@@ -708,6 +719,7 @@ static int ensure_matrix_setup(bosss_op* op) {
       bool dup = (c == j);
       for (int s2 = 1; s2 <= f && !dup; s2++) dup = (op->cols_host[(size_t)j * S + s2] == c);
       op->cols_host[(size_t)j * S + 1 + f] = dup ? -1 : c;
+      if (dup && c >= 0) op->merged_slots = true;
     }
   }
   // greedy distance-2 colouring of the cell graph
@@ -732,6 +744,20 @@ static int ensure_matrix_setup(bosss_op* op) {
   int rc;
   if ((rc = upload(&op->d_color, color.data(), color.size())) || (rc = upload(&op->d_cols, op->cols_host.data(), op->cols_host.size())))
     return rc;
+  return BOSSS_OK;
+}
+
+// Direct assembly of the linear forms (assemble_linear.hip): blocks of S slots per row, S = 1 the
+// diagonal alone.  The coefficient array is per operator and written by every call.
+static int assemble_linear(bosss_op* op, int S, double alpha, double beta, double shift, int transposed, double* blocks, hipStream_t s) {
+  const bosss_grid* g = op->grid;
+  if (!op->d_lincoef) HIPCHK(hipMalloc((void**)&op->d_lincoef, (size_t)g->J * linear_coefs_per_cell(op->D) * sizeof(double)));
+  LinArgs a;
+  a.J = g->J; a.detJ = g->detJ; a.invJ = g->invJ; a.scaling = g->scaling; a.lenscale = g->lenscale;
+  a.sqrtg = g->sqrtg; a.normal = g->normal; a.nb = g->nb; a.fp = op->fp;
+  launch_linear_assemble(op->kind == BOSSS_FORM_ADVDIFF, op->D, a, op->N, S, op->d_lintab, op->d_lincoef, alpha, beta, shift,
+                         transposed, blocks, s);
+  HIPCHK(hipGetLastError());
   return BOSSS_OK;
 }
 
@@ -826,9 +852,14 @@ int bosss_hip_op_assemble_dev(bosss_op* op, const double* U, double alpha, doubl
   if (op->precision != BOSSS_FP64) return fail(BOSSS_ERR_UNSUPPORTED, "assembly is FP64 only");
   int rc;
   HIPCHK(hipSetDevice(op->ctx->device));
-  if ((rc = ensure_matrix_setup(op)) || (rc = ensure_staging(op))) return rc;
+  if ((rc = ensure_matrix_setup(op))) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int J = op->grid->J, Nt = op->V * op->N, S = 1 + op->grid->NF;
+  // Linear forms: the blocks directly, unless a row reaches one cell across several faces (a
+  // periodic direction of one or two cells), whose blocks add up in one slot: those rows, and the
+  // Euler forms, go through the coloured probes.
+  if (op->d_lintab && !op->merged_slots) return assemble_linear(op, S, alpha, beta, 0.0, 0, blocks, s);
+  if ((rc = ensure_staging(op))) return rc;
   for (int k = 0; k < op->ncolors; k++)
     for (int q = 0; q < Nt; q++) {
       launch_probe(J, Nt, op->d_color, k, q, op->hX, s);
@@ -844,8 +875,9 @@ int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, doub
   if (!op || !U || !blocks) return fail(BOSSS_ERR_ARG, "NULL argument");
   int rc;
   HIPCHK(hipSetDevice(op->ctx->device));
-  if ((rc = ensure_staging(op))) return rc;
   hipStream_t s = (hipStream_t)stream;
+  if (op->d_lintab) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
+  if ((rc = ensure_staging(op))) return rc;
   const int J = op->grid->J, Nt = op->V * op->N;
   const size_t n = (size_t)J * Nt;
   const unsigned nb = (unsigned)((n + 255) / 256);
