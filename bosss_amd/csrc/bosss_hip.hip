@@ -68,6 +68,10 @@ struct bosss_grid {
   double* sqrtg;    // [J][NF]
   double* normal;   // [J][NF][D]
   int pair[6];
+  // axis-aligned cells (diagonal invJ, unit normals along the faces' axes): the same metrics in
+  // cell-fastest arrays, in one allocation each; nullptr otherwise
+  double* axis_real;   // [D][J] invJ diagonal, [NF][J] sqrtg
+  int* axis_nb;        // [NF][J]
 };
 
 struct bosss_op {
@@ -86,8 +90,10 @@ struct bosss_op {
   int ncolors;
   int32_t *d_color, *d_cols;
   std::vector<int32_t> cols_host;
-  // direct assembly of the linear forms: reference matrices (made at creation), per-cell coefficients
+  // direct assembly of the linear forms: host copy of the tables (vw, phi, dphi, fw, trace, dtrace),
+  // reference matrices (made from them on first use), per-cell coefficients
   bool merged_slots = false;   // a row holds one neighbour across several faces (or itself)
+  std::vector<double> lin_host;
   double *d_lintab = nullptr, *d_lincoef = nullptr;
   // tile shape of the block-ELL apply (panel size NL): tuned on the first device apply
   bool spmv_tuned = false;
@@ -107,6 +113,30 @@ void launch_bell_spmv(int J, int Nt, int S, const int32_t* cols, const double* b
                       double* y, hipStream_t s, int nl);
 int bell_default_nl(int Nt);
 void bell_candidates(int Nt, std::vector<int>& out);
+}
+
+// The cell-fastest copies of the metrics of an axis-aligned grid, made on the device from the
+// uploaded arrays.
+__global__ void __launch_bounds__(256) k_axis_arrays(int J, int D, const double* __restrict__ invJ, const double* __restrict__ sqrtg,
+                                                     const int* __restrict__ nb, double* __restrict__ real, int* __restrict__ anb) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x, NF = 2 * D;
+  if (j >= J) return;
+  for (int d = 0; d < D; d++) real[(size_t)d * J + j] = invJ[((size_t)j * D + d) * D + d];
+  for (int f = 0; f < NF; f++) {
+    real[(size_t)(D + f) * J + j] = sqrtg[(size_t)j * NF + f];
+    anb[(size_t)f * J + j] = nb[(size_t)j * NF + f];
+  }
+}
+static int make_axis_arrays(bosss_grid* G) {
+  const size_t J = G->J;
+  HIPCHK(hipMalloc((void**)&G->axis_real, (size_t)(G->D + G->NF) * J * sizeof(double)));
+  HIPCHK(hipMalloc((void**)&G->axis_nb, (size_t)G->NF * J * sizeof(int)));
+  hipStream_t s = G->ctx->stream;
+  hipLaunchKernelGGL(k_axis_arrays, dim3((unsigned)((J + 255) / 256)), dim3(256), 0, s, G->J, G->D, G->invJ, G->sqrtg, G->nb,
+                     G->axis_real, G->axis_nb);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(s));   // any stream may read them after the upload returns
+  return BOSSS_OK;
 }
 
 namespace bosss {
@@ -203,11 +233,36 @@ int bosss_hip_grid_upload(bosss_ctx* ctx, const bosss_grid_desc* g, bosss_grid**
   // carried by all but one layer of edges and the periodic wrap-arounds by one layer only, so
   // this is the stride of the slowest direction (a workgroup-ordering hint, no effect on results).
   std::map<int, int> offsets;
-  for (int e = 0; e < E; e++)
-    if (g->cells[2 * e + 1] >= 0) offsets[std::abs(g->cells[2 * e + 1] - g->cells[2 * e])]++;
+  int run_offset = -1, run = 0;   // edges of one direction come in runs of equal offset
+  for (int e = 0; e < E; e++) {
+    if (g->cells[2 * e + 1] < 0) continue;
+    const int o = std::abs(g->cells[2 * e + 1] - g->cells[2 * e]);
+    if (o != run_offset) {
+      if (run) offsets[run_offset] += run;
+      run_offset = o;
+      run = 0;
+    }
+    run++;
+  }
+  if (run) offsets[run_offset] += run;
   int plane = 0;
   for (const auto& oc : offsets)
     if (2LL * oc.second >= J) plane = std::max(plane, oc.first);
+
+  // Axis-aligned: invJ diagonal and positive, the normal of face f the unit vector of its axis and
+  // side, and opposite faces paired, on every cell.
+  bool axis = true;
+  for (int f = 0; f < NF && axis; f++) axis = face_dir(pair[f]) == face_dir(f) && face_upper(pair[f]) != face_upper(f);
+  for (int j = 0; j < J && axis; j++) {
+    for (int e = 0; e < D; e++)
+      for (int d = 0; d < D; d++) {
+        const double v = g->invJ[((size_t)j * D + e) * D + d];
+        axis = axis && (e == d ? v > 0.0 : v == 0.0);
+      }
+    for (int f = 0; f < NF; f++)
+      for (int d = 0; d < D; d++)
+        axis = axis && nrm[((size_t)j * NF + f) * D + d] == (d == face_dir(f) ? (face_upper(f) ? 1.0 : -1.0) : 0.0);
+  }
 
   HIPCHK(hipSetDevice(ctx->device));
   bosss_grid* G = new bosss_grid();
@@ -219,7 +274,7 @@ int bosss_hip_grid_upload(bosss_ctx* ctx, const bosss_grid_desc* g, bosss_grid**
   if ((rc = upload(&G->detJ, g->detJ, J)) || (rc = upload(&G->invJ, g->invJ, (size_t)J * D * D)) ||
       (rc = upload(&G->scaling, g->scaling, J)) || (rc = upload(&G->lenscale, g->lenscale, J)) ||
       (rc = upload(&G->nb, nb.data(), nb.size())) || (rc = upload(&G->sqrtg, sg.data(), sg.size())) ||
-      (rc = upload(&G->normal, nrm.data(), nrm.size()))) {
+      (rc = upload(&G->normal, nrm.data(), nrm.size())) || (axis && (rc = make_axis_arrays(G)))) {
     bosss_hip_grid_destroy(G);
     return rc;
   }
@@ -231,6 +286,7 @@ int bosss_hip_grid_destroy(bosss_grid* g) {
   if (!g) return BOSSS_OK;
   (void)hipFree(g->detJ); (void)hipFree(g->invJ); (void)hipFree(g->scaling); (void)hipFree(g->lenscale);
   (void)hipFree(g->nb); (void)hipFree(g->sqrtg); (void)hipFree(g->normal);
+  (void)hipFree(g->axis_real); (void)hipFree(g->axis_nb);
   delete g;
   return BOSSS_OK;
 }
@@ -438,9 +494,10 @@ int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tabl
     }
   }
   if (kind == BOSSS_FORM_SIP || kind == BOSSS_FORM_ADVDIFF) {
-    std::vector<double> T;
-    linear_reference_matrices(t->D, t->N, t->Kv, t->Ke, grid->pair, t->vol_weights, t->phi, t->dphi, t->face_weights, t->trace, t->dtrace, T);
-    if ((rc = upload(&op->d_lintab, T.data(), T.size()))) { bosss_hip_op_destroy(op); return rc; }
+    const size_t N = t->N, Kv = t->Kv, Ke = t->Ke, D = t->D, NF = 2 * D;
+    auto add = [&](const double* p, size_t n) { op->lin_host.insert(op->lin_host.end(), p, p + n); };
+    add(t->vol_weights, Kv); add(t->phi, Kv * N); add(t->dphi, Kv * N * D);
+    add(t->face_weights, Ke); add(t->trace, NF * Ke * N); add(t->dtrace, NF * Ke * N * D);
   }
   if ((rc = ks->prepare()) != 0) { bosss_hip_op_destroy(op); return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc); }
   *out = op;
@@ -514,10 +571,31 @@ static TArgs<Real> make_targs(const bosss_op* op, double alpha, double beta, con
   return a;
 }
 
+template <typename Real>
+static int launch_modal(const bosss_op* op, void (*k)(MArgs<Real>), double alpha, double beta, const void* U, const void* X, void* R,
+                        void* out, hipStream_t s) {
+  const bosss_grid* g = op->grid;
+  MArgs<Real> a;
+  a.J = g->J; a.nxcd = op->ctx->nxcd;
+  a.detJ = g->detJ; a.scaling = g->scaling; a.lenscale = g->lenscale;
+  a.g.iJ = g->axis_real; a.g.sqrtg = g->axis_real + (size_t)g->D * g->J; a.g.nb = g->axis_nb;
+  a.fp = op->fp; a.alpha = alpha; a.beta = beta;
+  a.U = (const Real*)U; a.X = (const Real*)X; a.R = (Real*)R; a.out = (Real*)out;
+  hipLaunchKernelGGL(k, dim3((unsigned)((g->J + 63) / 64)), dim3(64), 0, s, a);
+  HIPCHK(hipGetLastError());
+  return BOSSS_OK;
+}
+
 // own_only (JVP): the neighbour tangents are taken as zero, so the result is J(U)_jj X_j per cell.
 static int launch(bosss_op* op, int which, double alpha, double beta, const void* U, const void* X, void* R, void* out, hipStream_t s,
                   int own_only = 0) {
   HIPCHK(hipSetDevice(op->ctx->device));
+  // Linear scalar forms on axis-aligned cells: the modal kernels (own_only probes of these forms
+  // do not come here, their diagonal blocks are assembled directly).
+  if (op->tensor && op->grid->axis_nb && op->ks->km64[which] && !own_only) {
+    if (op->precision == BOSSS_FP64) return launch_modal<double>(op, op->ks->km64[which], alpha, beta, U, X, R, out, s);
+    if (op->ks->km32[which]) return launch_modal<float>(op, op->ks->km32[which], alpha, beta, U, X, R, out, s);
+  }
   if (op->tensor) {
     dim3 grid((op->grid->J + 16 * TWAVES - 1) / (16 * TWAVES)), block(64 * TWAVES);
     // Plane-fastest workgroup order (xcd_block) for the Euler JVP and VJP kernels when one
@@ -706,6 +784,17 @@ int bosss_hip_vjp(bosss_op* op, const double* U, const double* W, double* JtW) {
 }  // extern "C"
 
 // ------------------------------------------------------------------ matrix assembly
+// Reference matrices of a linear form, from the host copy of its tables.
+static int ensure_linear_tables(bosss_op* op) {
+  if (op->d_lintab) return BOSSS_OK;
+  const size_t N = op->N, D = op->D, NF = 2 * D, K1 = op->K1, Ke = D == 3 ? K1 * K1 : K1, Kv = Ke * K1;
+  const double* vw = op->lin_host.data();
+  const double *phi = vw + Kv, *dphi = phi + Kv * N, *fw = dphi + Kv * N * D, *tr = fw + Ke, *dtr = tr + NF * Ke * N;
+  std::vector<double> T;
+  linear_reference_matrices((int)D, (int)N, (int)Kv, (int)Ke, op->grid->pair, vw, phi, dphi, fw, tr, dtr, T);
+  return upload(&op->d_lintab, T.data(), T.size());
+}
+
 static int ensure_matrix_setup(bosss_op* op) {
   if (op->d_cols) return BOSSS_OK;
   const bosss_grid* g = op->grid;
@@ -742,6 +831,7 @@ static int ensure_matrix_setup(bosss_op* op) {
   }
   op->ncolors = ncol;
   int rc;
+  if (!op->lin_host.empty() && (rc = ensure_linear_tables(op))) return rc;
   if ((rc = upload(&op->d_color, color.data(), color.size())) || (rc = upload(&op->d_cols, op->cols_host.data(), op->cols_host.size())))
     return rc;
   return BOSSS_OK;
@@ -751,6 +841,7 @@ static int ensure_matrix_setup(bosss_op* op) {
 // diagonal alone.  The coefficient array is per operator and written by every call.
 static int assemble_linear(bosss_op* op, int S, double alpha, double beta, double shift, int transposed, double* blocks, hipStream_t s) {
   const bosss_grid* g = op->grid;
+  if (int rc = ensure_linear_tables(op)) return rc;
   if (!op->d_lincoef) HIPCHK(hipMalloc((void**)&op->d_lincoef, (size_t)g->J * linear_coefs_per_cell(op->D) * sizeof(double)));
   LinArgs a;
   a.J = g->J; a.detJ = g->detJ; a.invJ = g->invJ; a.scaling = g->scaling; a.lenscale = g->lenscale;
@@ -858,7 +949,7 @@ int bosss_hip_op_assemble_dev(bosss_op* op, const double* U, double alpha, doubl
   // Linear forms: the blocks directly, unless a row reaches one cell across several faces (a
   // periodic direction of one or two cells), whose blocks add up in one slot: those rows, and the
   // Euler forms, go through the coloured probes.
-  if (op->d_lintab && !op->merged_slots) return assemble_linear(op, S, alpha, beta, 0.0, 0, blocks, s);
+  if (!op->lin_host.empty() && !op->merged_slots) return assemble_linear(op, S, alpha, beta, 0.0, 0, blocks, s);
   if ((rc = ensure_staging(op))) return rc;
   for (int k = 0; k < op->ncolors; k++)
     for (int q = 0; q < Nt; q++) {
@@ -876,7 +967,7 @@ int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, doub
   int rc;
   HIPCHK(hipSetDevice(op->ctx->device));
   hipStream_t s = (hipStream_t)stream;
-  if (op->d_lintab) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
+  if (!op->lin_host.empty()) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
   if ((rc = ensure_staging(op))) return rc;
   const int J = op->grid->J, Nt = op->V * op->N;
   const size_t n = (size_t)J * Nt;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "dg_kernels.hpp"
+#include "dg_modal.hpp"
 #include "dg_tensor.hpp"
 
 namespace bosss {
@@ -23,6 +24,9 @@ struct KernelSet {
   void (*kt64[NVARIANT])(TArgs<double>);
   void (*kt32[NVARIANT])(TArgs<float>);
   size_t ktlds64[NVARIANT], ktlds32[NVARIANT];
+  // modal kernels (dg_modal.hpp) of the linear scalar forms on axis-aligned grids, or nullptr
+  void (*km64[NVARIANT])(MArgs<double>);
+  void (*km32[NVARIANT])(MArgs<float>);
   int prepare() const;
 };
 
@@ -52,6 +56,19 @@ void set_tensor_linearisations(void (**kt)(TArgs<Real>), size_t* lds) {
   }
 }
 
+template <class Form> struct ModalForm : std::false_type {};
+template <> struct ModalForm<FormSIP> : std::true_type {};
+template <> struct ModalForm<FormAdvDiff> : std::true_type {};
+
+template <class Form, int D, int P, typename Real>
+void set_modal(void (**km)(MArgs<Real>)) {
+  constexpr bool ADV = std::is_same<Form, FormAdvDiff>::value;
+  km[KernelSet::RES] = k_modal<D, P, Real, ADV, true, false, false>;
+  km[KernelSet::JVP] = k_modal<D, P, Real, ADV, true, true, false>;
+  km[KernelSet::VJP] = k_modal<D, P, Real, ADV, false, false, true>;
+  km[KernelSet::RES_VJP] = k_modal<D, P, Real, ADV, true, false, true>;
+}
+
 template <class Form, int D, int N, int K1, bool WITH32>
 KernelSet make_kernel_set(int kind) {
   typedef Shape<D, N, K1, Form::FACE_GRADU || Form::FACE_TESTG> S;
@@ -66,7 +83,10 @@ KernelSet make_kernel_set(int kind) {
   k.k64[KernelSet::JVP] = k_forward<Form, D, N, K1, double, MODE_JVP>;
   k.k64[KernelSet::VJP] = k_adjoint<Form, D, N, K1, double, false>;
   k.k64[KernelSet::RES_VJP] = k_adjoint<Form, D, N, K1, double, true>;
-  for (int i = 0; i < KernelSet::NVARIANT; i++) { k.k32[i] = nullptr; k.kt32[i] = nullptr; k.ktlds32[i] = 0; }
+  for (int i = 0; i < KernelSet::NVARIANT; i++) {
+    k.k32[i] = nullptr; k.kt32[i] = nullptr; k.ktlds32[i] = 0;
+    k.km64[i] = nullptr; k.km32[i] = nullptr;
+  }
   constexpr int P = degree_from_modes(D, N);
   static_assert(tdeg_count(D, P) == N, "N must be a full total-degree basis");
   typedef TShape<D, P, K1> TSh;
@@ -76,6 +96,11 @@ KernelSet make_kernel_set(int kind) {
   k.kt64[KernelSet::RES] = kt_forward<Form, D, P, K1, double, MODE_RES>;
   k.ktlds64[KernelSet::RES] = kt_forward_lds_bytes<Form, D, P, K1, double>(1);
   set_tensor_linearisations<Form, D, P, K1, double>(k.kt64, k.ktlds64);
+  if constexpr (ModalForm<Form>::value) {
+    static_assert(K1 >= P + 1, "the modal kernels replace a rule that is exact for products of two modes");
+    set_modal<Form, D, P, double>(k.km64);
+    if constexpr (WITH32) set_modal<Form, D, P, float>(k.km32);
+  }
   if constexpr (WITH32) {
     k.kt32[KernelSet::RES] = kt_forward<Form, D, P, K1, float, MODE_RES>;
     k.ktlds32[KernelSet::RES] = kt_forward_lds_bytes<Form, D, P, K1, float>(1);
