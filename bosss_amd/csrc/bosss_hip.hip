@@ -17,6 +17,7 @@
 #include "assemble_linear.hpp"
 #include "devbuf.hpp"
 #include "dg_kernels.hpp"
+#include "euler_blocks.hpp"
 #include "registry.hpp"
 
 using namespace bosss;
@@ -95,6 +96,9 @@ struct bosss_op {
   bool merged_slots = false;   // a row holds one neighbour across several faces (or itself)
   std::vector<double> lin_host;
   double *d_lintab = nullptr, *d_lincoef = nullptr;
+  // direct diagonal blocks of the Euler forms: tables, made on first use
+  double* d_ebreal = nullptr;
+  int32_t* d_ebints = nullptr;
   // tile shape of the block-ELL apply (panel size NL): tuned on the first device apply
   bool spmv_tuned = false;
   int spmv_nl = 0;
@@ -517,6 +521,8 @@ int bosss_hip_op_destroy(bosss_op* op) {
   if (op->d_first) (void)hipFree(op->d_first);
   if (op->d_lintab) (void)hipFree(op->d_lintab);
   if (op->d_lincoef) (void)hipFree(op->d_lincoef);
+  if (op->d_ebreal) (void)hipFree(op->d_ebreal);
+  if (op->d_ebints) (void)hipFree(op->d_ebints);
   delete op;
   return BOSSS_OK;
 }
@@ -852,6 +858,33 @@ static int assemble_linear(bosss_op* op, int S, double alpha, double beta, doubl
   return BOSSS_OK;
 }
 
+// Diagonal blocks of the Euler forms from moments of their flux Jacobians (euler_blocks.hip);
+// BOSSS_ERR_UNSUPPORTED where no such kernel is built.
+static int euler_blocks(bosss_op* op, const void* U, double alpha, double shift, int transposed, double* blocks, hipStream_t s) {
+  const bosss_grid* g = op->grid;
+  const int P = op->ks->P;
+  if (!op->d_ebreal) {
+    std::vector<double> x, w;
+    gauss_legendre(op->K1, x, w);
+    EulerBlockTables t;
+    euler_block_tables(op->D, P, op->K1, x, w, t);
+    int rc;
+    if ((!op->d_ebints && (rc = upload(&op->d_ebints, t.ints.data(), t.ints.size()))) ||
+        (rc = upload(&op->d_ebreal, t.real.data(), t.real.size())))
+      return rc;
+  }
+  EulerBlockArgs a;
+  a.J = g->J; a.detJ = g->detJ; a.invJ = g->invJ; a.scaling = g->scaling;
+  a.cf.nb = g->nb; a.cf.sqrtg = g->sqrtg; a.cf.normal = g->normal;
+  for (int f = 0; f < 6; f++) a.cf.pair[f] = g->pair[f];
+  a.fp = op->fp; a.real = op->d_ebreal; a.ints = op->d_ebints; a.U = U;
+  a.alpha = alpha; a.shift = shift; a.transposed = transposed; a.blocks = blocks;
+  if (!launch_euler_blocks(op->kind == BOSSS_FORM_EULER_HLLC, op->D, P, op->K1, op->precision == BOSSS_FP32, op->ctx->num_cu, a, s))
+    return BOSSS_ERR_UNSUPPORTED;
+  HIPCHK(hipGetLastError());
+  return BOSSS_OK;
+}
+
 // Diagonal cell blocks by probing the own-cell JVP: X[c][e] = (e == q) in every cell, then
 // blocks[j][r][q] = alpha * (J(U)_jj e_q)[r] + shift * (r == q)  (transposed: blocks[j][q][r], the
 // probe's column written contiguously; the row-major form writes it with a stride of Nt).
@@ -968,6 +1001,9 @@ int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, doub
   HIPCHK(hipSetDevice(op->ctx->device));
   hipStream_t s = (hipStream_t)stream;
   if (!op->lin_host.empty()) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
+  // Euler forms on tensor tables: directly, unless no kernel is built for them; operators on general
+  // tables go through the probes (20^3, p = 3: 17.4 ms by 100 probes, 1.18 ms directly).
+  if (op->tensor && (rc = euler_blocks(op, U, alpha, shift, (int)(transposed != 0), blocks, s)) != BOSSS_ERR_UNSUPPORTED) return rc;
   if ((rc = ensure_staging(op))) return rc;
   const int J = op->grid->J, Nt = op->V * op->N;
   const size_t n = (size_t)J * Nt;
