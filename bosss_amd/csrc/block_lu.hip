@@ -67,8 +67,8 @@ __device__ __forceinline__ void tile_load(double (&a)[RA][RA], const double* __r
   __syncthreads();
 }
 
-// Column steps 0..n-1 of getf2 (GJ = false) or of in-place Gauss-Jordan (GJ = true) on the register
-// tile.  Returns INFO (first zero pivot, 1-based; Gauss-Jordan stops there).  L.piv[j] receives the
+// Column steps 0..n-1 of getf2 on the register
+// tile.  Returns INFO (first zero pivot, 1-based).  L.piv[j] receives the
 // position of step j's pivot row, L.pos / L.lrow the final row placement (every wavefront's copy).
 //
 // One barrier per step: the 16 threads holding column j publish it and the pivot (row, value);
@@ -77,13 +77,13 @@ __device__ __forceinline__ void tile_load(double (&a)[RA][RA], const double* __r
 // Column group tc lives in wavefront tc / 4 and the LDS accesses of one wavefront complete in
 // order, so this exchange needs no workgroup barrier; lane 0 of each wavefront applies the row
 // exchange to that wavefront's copy of the placement.
-template <int RA, bool GJ>
+template <int RA>
 __device__ __forceinline__ int tile_eliminate(double (&a)[RA][RA], int n, TileLDS<RA>& L) {
   const int tid = threadIdx.x, tc = tid >> 4, tr = tid & 15, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   int* pos = L.pos[w];
   int* lrow = L.lrow[w];
-  unsigned used = 0;   // bit x: row tr + 16 x is in a position <= j (LU form only)
+  unsigned used = 0;   // bit x: row tr + 16 x is in a position <= j
   int inf = 0;
   for (int j = 0; j < n; j++) {
     const int k = j & 1, jc = j & 15, jy = j >> 4;
@@ -107,7 +107,6 @@ __device__ __forceinline__ int tile_eliminate(double (&a)[RA][RA], int n, TileLD
                 if (v > best || (v == best && ps < bpos)) { best = v; bpos = ps; bp = r; bval = v0; }
               }
             }
-            if (GJ) a[x][yy] = 0.0;   // becomes -a[r][j] / pivot through the update
           }
         }
 #pragma unroll
@@ -128,7 +127,6 @@ __device__ __forceinline__ int tile_eliminate(double (&a)[RA][RA], int n, TileLD
     if (tid == 0) L.piv[j] = pos[p];
     if (!(pv != 0.0)) {   // zero pivot (NaN passes, as in DGETF2)
       if (!inf) inf = j + 1;
-      if (GJ) return inf;
       const int r0 = lrow[j];   // no exchange: the row in position j is done all the same
       if (tr == (r0 & 15)) used |= 1u << (r0 >> 4);
       continue;
@@ -146,7 +144,7 @@ __device__ __forceinline__ int tile_eliminate(double (&a)[RA][RA], int n, TileLD
 #pragma unroll
           for (int y = 0; y < RA; y++) {
             const int c = tc + 16 * y;
-            L.row[k][c] = GJ ? (c == j ? pinv : a[xx][y] * pinv) : a[xx][y];
+            L.row[k][c] = a[xx][y];
           }
         }
     }
@@ -154,49 +152,30 @@ __device__ __forceinline__ int tile_eliminate(double (&a)[RA][RA], int n, TileLD
     double u[RA];
 #pragma unroll
     for (int y = 0; y < RA; y++) u[y] = L.row[k][tc + 16 * y];
-    if (GJ) {
+    // rows after the pivot in factor order: multiplier into column j, columns > j updated
 #pragma unroll
-      for (int x = 0; x < RA; x++) {
-        const int r = tr + 16 * x;
-        const double f = r < n ? L.col[k][r] : 0.0;
+    for (int x = 0; x < RA; x++) {
+      const int r = tr + 16 * x;
+      if (r < n && r != p && !((used >> x) & 1u)) {
+        const double l = L.col[k][r] * pinv;
 #pragma unroll
-        for (int y = 0; y < RA; y++) a[x][y] -= f * u[y];
-      }
-      if (tr == pc) {
+        for (int y = 0; y < RA; y++)
+          if (tc + 16 * y > j) a[x][y] -= l * u[y];
+        if (tc == jc) {
 #pragma unroll
-        for (int xx = 0; xx < RA; xx++)
-          if (xx == px) {
-#pragma unroll
-            for (int y = 0; y < RA; y++) a[xx][y] = u[y];
-          }
-      }
-    } else {
-      // rows after the pivot in factor order: multiplier into column j, columns > j updated
-#pragma unroll
-      for (int x = 0; x < RA; x++) {
-        const int r = tr + 16 * x;
-        if (r < n && r != p && !((used >> x) & 1u)) {
-          const double l = L.col[k][r] * pinv;
-#pragma unroll
-          for (int y = 0; y < RA; y++)
-            if (tc + 16 * y > j) a[x][y] -= l * u[y];
-          if (tc == jc) {
-#pragma unroll
-            for (int yy = 0; yy < RA; yy++)
-              if (yy == jy) a[x][yy] = l;
-          }
+          for (int yy = 0; yy < RA; yy++)
+            if (yy == jy) a[x][yy] = l;
         }
       }
-      if (tr == pc) used |= 1u << px;
     }
+    if (tr == pc) used |= 1u << px;
   }
   return inf;
 }
 
-// Writes the tile back: factors in position order (row pos[r]), or the inverse with the column
-// permutation too (X[pos[r]][lrow[c]] = a[r][c]).
+// Writes the factors back in position order (row pos[r]).
 template <int RA>
-__device__ __forceinline__ void tile_store(const double (&a)[RA][RA], double* __restrict__ g, int n, const TileLDS<RA>& L, bool inverse) {
+__device__ __forceinline__ void tile_store(const double (&a)[RA][RA], double* __restrict__ g, int n, const TileLDS<RA>& L) {
   const int tid = threadIdx.x, tc = tid >> 4, tr = tid & 15;
 #pragma unroll
   for (int x = 0; x < RA; x++) {
@@ -206,16 +185,13 @@ __device__ __forceinline__ void tile_store(const double (&a)[RA][RA], double* __
 #pragma unroll
       for (int y = 0; y < RA; y++) {
         const int c = tc + 16 * y;
-        if (c < n) g[row + (inverse ? L.lrow[0][c] : c)] = a[x][y];
+        if (c < n) g[row + c] = a[x][y];
       }
     }
   }
 }
 
-// Waves per SIMD the register-tile kernel is compiled for.  The 100-DOF blocks (RA = 7) with the
-// inverse need 186 VGPRs unconstrained (two waves); at three waves (168 VGPRs, an 88 B per-lane
-// spill) the 262 144 blocks of p = 3 Euler factor and invert in 95 ms instead of 122 ms, the
-// column steps being latency bound (four waves spill 240 B and take 329 ms).
+// Waves per SIMD the register-tile kernel is compiled for: the column steps are latency bound.
 template <int RA>
 constexpr int lu_tile_waves() { return RA == 7 ? 3 : 1; }
 
@@ -229,14 +205,9 @@ constexpr int lu_tile_waves() { return RA == 7 ? 3 : 1; }
 // group and publish the column; the threads holding the pivot row publish it to their own
 // 16-lane groups; every thread updates its entries.  Factors, pivots and INFO are getf2's, operation for operation (multiplier a * (1 / pivot),
 // then the rank-one update of the columns after j).
-//
-// With INV the elimination is Gauss-Jordan in place (every row other than the pivot row updated at
-// every step: uniform work for all threads) and the inverse is written out with the row and column
-// permutation applied.  A zero pivot stops it; the block is then factored from its original values
-// instead (LU factors and INFO, no inverse, as DGETRF leaves them when DGETRI cannot proceed).  Register columns and rows are
-// picked with wavefront-uniform branches, so no register array is indexed dynamically (the block
-// stays in registers; RA = 7 with the inverse spills 88 B per lane at the three waves above).
-template <int RA, bool INV>
+// Register columns and rows are picked with wavefront-uniform branches, so no register array is
+// indexed dynamically.
+template <int RA>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lu_tile_waves<RA>()))) k_block_lu_tile(int nblk, int nmax, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
                                                        double* __restrict__ A, int32_t* __restrict__ ipiv,
                                                        const int64_t* __restrict__ pivoff, int32_t* __restrict__ info) {
@@ -251,21 +222,318 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lu_til
   double* g = A + off[b];
   double a[RA][RA];
   tile_load<RA>(a, g, n, L);
-  int inf = 0;
-  bool inverse = false;
-  if (INV) {
-    inf = tile_eliminate<RA, true>(a, n, L);
-    inverse = inf == 0;
-    if (!inverse) {   // singular: factor the original block (LU and INFO, no inverse)
-      __syncthreads();
-      tile_load<RA>(a, g, n, L);
-    }
-  }
-  if (!inverse) inf = tile_eliminate<RA, false>(a, n, L);
+  const int inf = tile_eliminate<RA>(a, n, L);
   __syncthreads();
-  tile_store<RA>(a, g, n, L, inverse);
+  tile_store<RA>(a, g, n, L);
   if (ipiv)
     for (int i = threadIdx.x; i < n; i += 256) ipiv[pivoff[b] + i] = L.piv[i] + 1;
+  if (threadIdx.x == 0 && info) info[b] = inf;
+}
+
+// Inverse of blocks of 21..128 DOF, blocked: Gauss-Jordan on panels of four columns, the rest of
+// the block updated by one rank-4 product per panel on v_mfma_f64_16x16x4f64.
+//
+// One workgroup of four wavefronts per block, the block in registers as 16 x 16 accumulator tiles:
+// wavefront w holds tile columns w and w + 4 (TR tile rows each), rows in their original places
+// (row exchanges are bookkeeping, as in the register-tile form).  Per panel the wavefront that holds
+// its four columns runs in-place Gauss-Jordan on them, lane l with rows l and l + 64: pivots are
+// getf2's (largest |a| among the rows not yet used, ties to the smaller position, a NaN in position j
+// never beaten) on columns updated by the earlier panels.  The other columns then receive the same four
+// steps: the scaled pivot rows u_0 .. u_3 are formed one after the other (u_k = (a_pk - sum_i<k f_i(p_k) u_i)
+// / pivot k, f_i(r) the entry of row r in column i before step i) and all rows take -sum_k f_k(r) u_k, a
+// pivot row from zero on and with 1 in its own step.  Same operations in the same order as column by
+// column; the rank-4 form X = -A_RJ A_PJ^-1, A += X A_P has larger coefficients and measured 1.8 times
+// the error.  One barrier per panel (X, F double-buffered): pivot rows are exchanged inside the
+// wavefront that owns their columns.
+//
+// Bound: the latency of the panel's four column steps, which one wavefront runs; three workgroups per
+// CU overlap it (100 DOF: two waves per SIMD 1.27 ms, three 0.92 ms).  4000 blocks of 100 DOF: 1.61 ms
+// column by column in a register tile (260 vector and 34 LDS instructions per wavefront and column),
+// 0.92 ms here; 32 DOF 134 -> 122 us, 64 DOF 0.43 -> 0.31 ms, 128 DOF 2.77 -> 1.50 ms.  The results
+// are those of the column-by-column form to the bit.
+// A zero pivot stops it and the block is factored from its original values instead (LU and INFO).
+typedef double gj_f64x4 __attribute__((ext_vector_type(4)));
+
+// Maximum over the 64 lanes of values that are not NaN, the same in every lane.
+__device__ __forceinline__ double wave_max(double v) {
+  auto step = [](double x, auto ctrl, auto mask) {
+    union { double d; int i[2]; } u, t;
+    u.d = x;
+    t.i[0] = __builtin_amdgcn_update_dpp(u.i[0], u.i[0], decltype(ctrl)::value, decltype(mask)::value, 0xf, false);
+    t.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], decltype(ctrl)::value, decltype(mask)::value, 0xf, false);
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(t.d));   // fmax() would quiet both operands first
+    return r;
+  };
+  v = step(v, std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xf>());   // row_shr:1
+  v = step(v, std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xf>());   // row_shr:2
+  v = step(v, std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xf>());   // row_shr:4
+  v = step(v, std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xf>());   // row_shr:8
+  v = step(v, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());   // row_bcast:15
+  v = step(v, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());   // row_bcast:31
+  union { double d; int i[2]; } r;
+  r.d = v;
+  r.i[0] = __builtin_amdgcn_readlane(r.i[0], 63);
+  r.i[1] = __builtin_amdgcn_readlane(r.i[1], 63);
+  return r.d;
+}
+__device__ __forceinline__ double wave_read(double v, int lane) {   // lane: wavefront-uniform
+  union { double d; int i[2]; } u;
+  u.d = v;
+  u.i[0] = __builtin_amdgcn_readlane(u.i[0], lane);
+  u.i[1] = __builtin_amdgcn_readlane(u.i[1], lane);
+  return u.d;
+}
+
+template <int TR>
+struct PanelLDS {
+  double X[2][16 * TR][4];       // the panel before and after its column steps
+  double F[2][16 * TR][4];       // coefficient of pivot row k in every row's update
+  double tri[2][4][4];           // [k][i < k]: pivot row k's entry in column i before step i; [k][k]: 1 / pivot k
+  double row[4][4][32];          // per wavefront: the four pivot rows at its columns
+  int pos[16 * TR], row_at[16 * TR], piv[16 * TR], p[2][4], stop[2];
+};
+
+// Column steps j0 .. j0 + nb - 1 (nb <= 4) on the panel in X, by one wavefront.  Returns 0 or
+// INFO at a zero pivot; p[k] receives the pivot row of step k, F and tri its update (see gj_blocked).
+template <int TR>
+__device__ __forceinline__ int gj_panel(double (*X)[4], double (*F)[4], double (*tri)[4], int n, int j0, int nb, int* pos_, int* piv, int* p_) {
+  const int lane = threadIdx.x & 63;
+  const int r1 = lane + 64 < 16 * TR ? lane + 64 : 16 * TR - 1;   // rows of this lane; lanes past the tile hold no second row
+  const bool in0 = lane < n, in1 = lane + 64 < 16 * TR && lane + 64 < n;
+  double v[2][4], f[2][4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    f[0][k] = f[1][k] = 0.0;
+    v[0][k] = lane < 16 * TR ? X[lane < 16 * TR ? lane : 0][k] : 0.0;
+    v[1][k] = X[r1][k];
+  }
+  int pos0 = lane < 16 * TR ? pos_[lane < 16 * TR ? lane : 0] : -1, pos1 = in1 ? pos_[r1] : -1;
+#pragma unroll
+  for (int jj = 0; jj < 4; jj++) {
+    if (jj >= nb) break;
+    const int j = j0 + jj;
+    auto cand = [&](double x, int ps, bool in) {
+      double c = fabs(x);
+      if (c != c) c = ps == j ? (double)INFINITY : -1.0;   // idamax: a NaN first element is never beaten, any other never chosen
+      return in && ps >= j ? c : -1.0;
+    };
+    const double c0 = cand(v[0][jj], pos0, in0), c1 = cand(v[1][jj], pos1, in1);
+    const double best = wave_max(c0 > c1 ? c0 : c1);
+    // rows holding the maximum (the row in position j always qualifies for best >= 0); ties to the smaller position
+    unsigned long long m0 = __ballot(c0 == best), m1 = __ballot(c1 == best);
+    int p = m0 ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
+    int q = p < 64 ? __builtin_amdgcn_readlane(pos0, p) : __builtin_amdgcn_readlane(pos1, p - 64);
+    if (__builtin_popcountll(m0) + __builtin_popcountll(m1) > 1) {
+      while (m0) {
+        const int r = __builtin_ctzll(m0), ps = __builtin_amdgcn_readlane(pos0, r);
+        m0 &= m0 - 1;
+        if (ps < q) { q = ps; p = r; }
+      }
+      while (m1) {
+        const int r = __builtin_ctzll(m1), ps = __builtin_amdgcn_readlane(pos1, r);
+        m1 &= m1 - 1;
+        if (ps < q) { q = ps; p = 64 + r; }
+      }
+    }
+    p = __builtin_amdgcn_readfirstlane(p);
+    q = __builtin_amdgcn_readfirstlane(q);
+    const int pl = p & 63;
+    double u[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) u[k] = wave_read(p < 64 ? v[0][k] : v[1][k], pl);
+    if (!(u[jj] != 0.0)) return j + 1;   // NaN passes, as in DGETF2
+    // exchange of positions: the row in position j goes to the pivot row's place
+    if (pos0 == j) pos0 = q;
+    if (pos1 == j) pos1 = q;
+    if (lane == pl) { if (p < 64) pos0 = j; else pos1 = j; }
+    const double pinv = 1.0 / u[jj];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (i < jj) {
+        const double t = wave_read(p < 64 ? f[0][i] : f[1][i], pl);
+        if (lane == 0) tri[jj][i] = -t;
+      }
+    if (lane == 0) { piv[j] = q; p_[jj] = p; tri[jj][jj] = pinv; }
+#pragma unroll
+    for (int k = 0; k < 4; k++) u[k] = k == jj ? pinv : u[k] * pinv;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const bool self = lane == pl && (p >> 6) == h;
+      const double m = v[h][jj];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (i < jj) f[h][i] = self ? 0.0 : f[h][i];
+      f[h][jj] = self ? 1.0 : -m;
+      v[h][jj] = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[h][k] = self ? u[k] : v[h][k] - m * u[k];
+    }
+  }
+  if (lane < 16 * TR) {
+    pos_[lane] = pos0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) { X[lane][k] = v[0][k]; F[lane][k] = f[0][k]; }
+  }
+  if (lane + 64 < 16 * TR) {
+    if (in1) pos_[r1] = pos1;
+#pragma unroll
+    for (int k = 0; k < 4; k++) { X[r1][k] = v[1][k]; F[r1][k] = f[1][k]; }
+  }
+  return 0;
+}
+
+// In-place inverse of the n x n block g, n <= 16 TR; returns 0, or INFO with g untouched.
+template <int TR>
+__device__ __forceinline__ int gj_blocked(double* __restrict__ g, int n, PanelLDS<TR>& L) {
+  constexpr int TC = (TR + 3) / 4;      // tile columns of a wavefront: w, w + 4
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  gj_f64x4 a[TC][TR];
+#pragma unroll
+  for (int c = 0; c < TC; c++)
+#pragma unroll
+    for (int t = 0; t < TR; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int row = 16 * t + grp + 4 * r, cc = 16 * (w + 4 * c) + col;
+        a[c][t][r] = row < n && cc < n ? g[(int64_t)row * n + cc] : 0.0;
+      }
+  for (int i = tid; i < 16 * TR; i += 256) L.pos[i] = i;
+  __syncthreads();
+  for (int j0 = 0, k = 0; j0 < n; j0 += 4, k ^= 1) {
+    const int nb = n - j0 < 4 ? n - j0 : 4;
+    const int tc = j0 >> 4, cs = tc >> 2, c4 = (j0 & 15) >> 2;   // tile column of the panel, its slot, the lanes' column group
+    double (*X)[4] = L.X[k];
+    if ((tc & 3) == w) {
+      const int kc = col & 3;
+      if ((col >> 2) == c4) {
+#pragma unroll
+        for (int c = 0; c < TC; c++)
+          if (c == cs) {
+#pragma unroll
+            for (int t = 0; t < TR; t++)
+#pragma unroll
+              for (int r = 0; r < 4; r++) X[16 * t + grp + 4 * r][kc] = a[c][t][r];
+          }
+      }
+      __builtin_amdgcn_wave_barrier();
+      const int inf = gj_panel<TR>(X, L.F[k], L.tri[k], n, j0, nb, L.pos, L.piv, L.p[k]);
+      if (lane == 0) L.stop[k] = inf;
+    }
+    __syncthreads();
+    const int stop = __builtin_amdgcn_readfirstlane(L.stop[k]);
+    if (stop) return stop;
+    // pivot rows at this wavefront's columns: out to LDS, zero in the tiles
+    double (*P)[32] = L.row[w];
+    for (int q = 0; q < nb; q++) {
+      const int p = __builtin_amdgcn_readfirstlane(L.p[k][q]);
+#pragma unroll
+      for (int t = 0; t < TR; t++)
+        if (t == (p >> 4)) {
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if (r == ((p >> 2) & 3)) {
+              const bool mine = grp == (p & 3);
+              if constexpr (TR == 7) {   // at three waves per SIMD the selects below spill (100 DOF: +8 %; other sizes -5 %)
+                if (mine)
+#pragma unroll
+                  for (int c = 0; c < TC; c++) { P[q][16 * c + col] = a[c][t][r]; a[c][t][r] = 0.0; }
+              } else {
+#pragma unroll
+                for (int c = 0; c < TC; c++) {
+                  if (mine) P[q][16 * c + col] = a[c][t][r];
+                  a[c][t][r] = mine ? 0.0 : a[c][t][r];
+                }
+              }
+            }
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    double b[TC], x[TR], tri[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int i = 0; i <= q; i++) tri[q][i] = q < nb ? L.tri[k][q][i] : 0.0;
+#pragma unroll
+    for (int c = 0; c < TC; c++) {
+      double u[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {      // steps past nb have tri = 0
+        u[q] = q < nb ? P[q][16 * c + col] : 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (i < q) u[q] -= tri[q][i] * u[i];
+        u[q] *= tri[q][q];
+      }
+      b[c] = grp == 0 ? u[0] : grp == 1 ? u[1] : grp == 2 ? u[2] : u[3];
+    }
+#pragma unroll
+    for (int t = 0; t < TR; t++) x[t] = L.F[k][16 * t + col][grp];
+#pragma unroll
+    for (int c = 0; c < TC; c++)
+      if (w + 4 * c < TR)
+#pragma unroll
+        for (int t = 0; t < TR; t++) a[c][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], b[c], a[c][t], 0, 0, 0);
+    if ((tc & 3) == w && (col >> 2) == c4 && (col & 3) < nb) {   // the panel's own columns
+#pragma unroll
+      for (int c = 0; c < TC; c++)
+        if (c == cs) {
+#pragma unroll
+          for (int t = 0; t < TR; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) a[c][t][r] = X[16 * t + grp + 4 * r][col & 3];
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  // X[pos[r]][row placed in position c] = a[r][c]
+  for (int i = tid; i < n; i += 256) L.row_at[L.pos[i]] = i;
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < TR; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = 16 * t + grp + 4 * r;
+      if (row < n) {
+        const int64_t o = (int64_t)L.pos[row] * n;
+#pragma unroll
+        for (int c = 0; c < TC; c++) {
+          const int cc = 16 * (w + 4 * c) + col;
+          if (cc < n) g[o + L.row_at[cc]] = a[c][t][r];
+        }
+      }
+    }
+  return 0;
+}
+
+template <int TR>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TR <= 4 ? 4 : TR == 7 ? 3 : 2))) k_block_inverse(int nblk, int nmax, const int32_t* __restrict__ nsz,
+                                                                const int64_t* __restrict__ off, double* __restrict__ A,
+                                                                int32_t* __restrict__ ipiv, const int64_t* __restrict__ pivoff,
+                                                                int32_t* __restrict__ info) {
+  __shared__ union { PanelLDS<TR> panel; TileLDS<TR> tile; } L;
+  const int b = blockIdx.x;
+  if (b >= nblk) return;
+  const int n = nsz[b];
+  if (n <= 0 || n > nmax || n > 16 * TR) {   // size outside what the launch was sized for: report, touch nothing
+    if (threadIdx.x == 0 && info) info[b] = -1;
+    return;
+  }
+  double* g = A + off[b];
+  int inf = gj_blocked<TR>(g, n, L.panel);
+  const int* piv = L.panel.piv;
+  if (inf) {   // singular: factor the original block (LU and INFO, no inverse)
+    __syncthreads();
+    double a[TR][TR];
+    tile_load<TR>(a, g, n, L.tile);
+    inf = tile_eliminate<TR>(a, n, L.tile);
+    __syncthreads();
+    tile_store<TR>(a, g, n, L.tile);
+    piv = L.tile.piv;
+  }
+  if (ipiv)
+    for (int i = threadIdx.x; i < n; i += 256) ipiv[pivoff[b] + i] = piv[i] + 1;
   if (threadIdx.x == 0 && info) info[b] = inf;
 }
 
@@ -773,9 +1041,9 @@ static int lu_launch_reg(int nblk, int nmax, const int32_t* n, const int64_t* of
   const dim3 grid((unsigned)nblk), blk(256);
 #define LU_TILE(RA)                                                                                                     \
   if (want_inverse)                                                                                                     \
-    hipLaunchKernelGGL((k_block_lu_tile<RA, true>), grid, blk, 0, s, nblk, nmax, n, off, A, ipiv, pivoff, info);        \
+    hipLaunchKernelGGL(k_block_inverse<RA>, grid, blk, 0, s, nblk, nmax, n, off, A, ipiv, pivoff, info);                \
   else                                                                                                                  \
-    hipLaunchKernelGGL((k_block_lu_tile<RA, false>), grid, blk, 0, s, nblk, nmax, n, off, A, ipiv, pivoff, info);
+    hipLaunchKernelGGL(k_block_lu_tile<RA>, grid, blk, 0, s, nblk, nmax, n, off, A, ipiv, pivoff, info);
   if (nmax <= 32) {
     LU_TILE(2)
   } else if (nmax <= 64) {
