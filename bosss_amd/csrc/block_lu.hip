@@ -13,6 +13,7 @@
 // of uneven XDG blocks (10x10 and 20x20) is one kernel.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <mutex>
@@ -275,6 +276,26 @@ __device__ __forceinline__ double wave_max(double v) {
   r.d = v;
   r.i[0] = __builtin_amdgcn_readlane(r.i[0], 63);
   r.i[1] = __builtin_amdgcn_readlane(r.i[1], 63);
+  return r.d;
+}
+// Maximum of lanes 0..7, in every lane.
+__device__ __forceinline__ double wave_max8(double v) {
+  auto step = [](double x, auto ctrl) {
+    union { double d; int i[2]; } u, t;
+    u.d = x;
+    t.i[0] = __builtin_amdgcn_update_dpp(u.i[0], u.i[0], decltype(ctrl)::value, 0xf, 0xf, false);
+    t.i[1] = __builtin_amdgcn_update_dpp(u.i[1], u.i[1], decltype(ctrl)::value, 0xf, 0xf, false);
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(t.d));
+    return r;
+  };
+  v = step(v, std::integral_constant<int, 0x111>());
+  v = step(v, std::integral_constant<int, 0x112>());
+  v = step(v, std::integral_constant<int, 0x114>());
+  union { double d; int i[2]; } r;
+  r.d = v;
+  r.i[0] = __builtin_amdgcn_readlane(r.i[0], 7);
+  r.i[1] = __builtin_amdgcn_readlane(r.i[1], 7);
   return r.d;
 }
 __device__ __forceinline__ double wave_read(double v, int lane) {   // lane: wavefront-uniform
@@ -892,46 +913,482 @@ __global__ void k_lu_info(int nblk, const int32_t* __restrict__ st, int32_t* __r
 }
 
 
-// x_b <- LU_b \ x_b   (getrs with the 1-based pivots), one wavefront per block, any size up to
-// 4096.  Lane l owns the rows i = l (mod 64) of x_b and is the only one to write them: the
-// substitutions run column by column, the finished x_j reaches the other lanes by a shuffle from
-// its owner, and each owner subtracts L_ij x_j (U_ij x_j) from its rows.  The forward sweep adds
-// the terms of a row in getrs' order (k = 0 .. i-1), the backward sweep from the last column.
-template <typename Real>
-__global__ void __launch_bounds__(64) k_block_solve(int nblk, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
-                                                    const Real* __restrict__ LU, const int32_t* __restrict__ ipiv,
-                                                    const int64_t* __restrict__ pivoff, const int64_t* __restrict__ xoff,
-                                                    Real* __restrict__ x) {
+// Blocks of 129..LU_REG_MAXN DOF whose pivots the caller keeps: the panel in registers, two launches
+// per panel and nothing else kept between them (a zero-pivot column is one whose diagonal is zero).
+//
+// k_lu_panel_reg: one workgroup of 512 threads per block, thread t holds the panel rows k0 + t and
+// k0 + 512 + t (32 columns each).  A column step is a wavefront maximum, one exchange of the eight
+// wavefront winners and one of the pivot row through LDS (two barriers), and the rank-one update of
+// the panel in registers; the panel's columns are walked in four groups of eight that rotate through
+// the same registers, so the loop body stays small.  Operations and order are getf2's.
+// k_lu_update: one workgroup per 32 columns outside the panel applies the panel's 32 row exchanges
+// (as one permutation, every value read before any is written), and to the right of the panel the
+// solve with L11 and the product A22 -= L21 U12 on the matrix units.
+//
+// Bound: the latency of the column steps (1.5 us each at 500 rows, 0.8 us below 256; 4.6 us in the form
+// that searches, swaps and updates in global memory, k_lu_panel).  48 blocks of 200..540 DOF, factored:
+// 3.4 ms before, 1.3 ms here; 300 of 200 1.07 -> 0.58 ms, 300 of 1024 67 -> 22 ms; factors and pivots the
+// same to the bit.  Measured and not kept: the panel rows turned through LDS for coalesced access
+// (48 -> 56 us per panel), exchanged rows moved between threads instead of their positions (64 us).
+constexpr int LU_REG_MAXN = 1024, LU_COLS = 32;
+
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) k_lu_panel_reg(int k0, int nblk, int nmax, const int32_t* __restrict__ nsz,
+                                                          const int64_t* __restrict__ off, double* __restrict__ A,
+                                                          int32_t* __restrict__ piv, const int64_t* __restrict__ pivoff) {
+  constexpr int W = THREADS / 64;
+  static_assert(W == 4 || W == 8, "the winners of the wavefronts are reduced over eight lanes");
+  __shared__ double s_val[2][8];
+  __shared__ int s_pos[2][8];
+  __shared__ __align__(16) double s_piv[2][LU_NB];
   const int b = blockIdx.x;
   if (b >= nblk) return;
   const int n = nsz[b];
-  if (n <= 0) return;
+  if (n <= 0 || n > nmax || k0 >= n || n - k0 > 2 * THREADS) return;   // (the launch's thread count covers nmax)
+  double* a = A + off[b] + k0;
+  int32_t* pb = piv + pivoff[b] + k0;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nb = n - k0 < LU_NB ? n - k0 : LU_NB;
+  // rows stay with their threads; pos is the position (row of the factors) the exchanges have given them
+  int pos[2] = {k0 + t, k0 + THREADS + t};
+  const bool two = k0 + THREADS < n, in[2] = {pos[0] < n, pos[1] < n};
+  double v[2][LU_NB];
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int c = 0; c < LU_NB; c++) v[h][c] = in[h] && c < nb ? a[(size_t)pos[h] * n + c] : 0.0;
+  if (t < 16) { s_val[t >> 3][t & 7] = -1.0; s_pos[t >> 3][t & 7] = 1 << 30; }
+  __syncthreads();
+#pragma unroll 1
+  for (int s = 0; s < LU_NB / 8; s++) {
+#pragma unroll
+    for (int jj = 0; jj < 8; jj++) {
+      const int jl = 8 * s + jj, j = k0 + jl, k = jj & 1;
+      if (jl < nb) {
+        auto cand = [&](double x, int ps, bool ok) {
+          double c = fabs(x);
+          if (c != c) c = ps == j ? (double)INFINITY : -1.0;   // idamax: a NaN first element is never beaten, any other never chosen
+          return ok && ps >= j ? c : -1.0;
+        };
+        const double c0 = cand(v[0][jj], pos[0], in[0]), c1 = two ? cand(v[1][jj], pos[1], in[1]) : -1.0;
+        const double best = wave_max(c0 > c1 ? c0 : c1);
+        // smallest position among the rows holding the maximum
+        auto first = [&](unsigned long long m, int ps) {
+          int r = 1 << 30;
+          for (; m; m &= m - 1) r = std::min(r, __builtin_amdgcn_readlane(ps, __builtin_ctzll(m)));
+          return r;
+        };
+        if (best >= 0.0) {
+          int q = first(__ballot(c0 == best), pos[0]);
+          if (two) q = std::min(q, first(__ballot(c1 == best), pos[1]));
+          if (lane == 0) { s_val[k][w] = best; s_pos[k][w] = q; }
+        } else if (lane == 0) {
+          s_val[k][w] = -1.0;
+        }
+        __syncthreads();
+        const double bv = s_val[k][lane & 7];
+        const int bp = s_pos[k][lane & 7];
+        const int q = __builtin_amdgcn_readfirstlane(first(__ballot(bv == wave_max8(bv)) & 0xff, bp));   // the row in position j always takes part
+        if (pos[0] == q)
+#pragma unroll
+          for (int c = 0; c < LU_NB; c++) s_piv[k][c] = v[0][c];
+        if (two && pos[1] == q)
+#pragma unroll
+          for (int c = 0; c < LU_NB; c++) s_piv[k][c] = v[1][c];
+        if (t == 0) pb[jl] = q + 1;
+        __syncthreads();
+        const double pv = s_piv[k][jj];
+        if (pv != 0.0) {   // NaN passes, as in DGETF2; a zero pivot leaves the column as it is
+#pragma unroll
+          for (int h = 0; h < 2; h++) pos[h] = pos[h] == q ? j : (pos[h] == j ? q : pos[h]);
+          const double inv = 1.0 / pv;
+          const bool act[2] = {in[0] && pos[0] > j, in[1] && pos[1] > j};
+          double l[2];
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            l[h] = v[h][jj] * inv;
+            if (act[h]) v[h][jj] = l[h];
+          }
+#pragma unroll
+          for (int g = 0; g < LU_NB / 8; g++)
+            if (g == 0 || s < LU_NB / 8 - g) {   // column groups still to be factored
+              double u[8];
+#pragma unroll
+              for (int c = 0; c < 8; c++) u[c] = s_piv[k][8 * g + c];
+              if (act[0])
+#pragma unroll
+                for (int c = g == 0 ? jj + 1 : 0; c < 8; c++) v[0][8 * g + c] -= l[0] * u[c];
+              if (two && act[1])
+#pragma unroll
+                for (int c = g == 0 ? jj + 1 : 0; c < 8; c++) v[1][8 * g + c] -= l[1] * u[c];
+            }
+        }
+      }
+    }
+    // the next eight columns move to the front
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int c = 0; c < 8; c++) {
+        const double x = v[h][c];
+        v[h][c] = v[h][c + 8];
+        v[h][c + 8] = v[h][c + 16];
+        v[h][c + 16] = v[h][c + 24];
+        v[h][c + 24] = x;
+      }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+    if (in[h])
+#pragma unroll
+      for (int c = 0; c < LU_NB; c++)
+        if (c < nb) a[(size_t)pos[h] * n + c] = v[h][c];
+}
+
+__global__ void __launch_bounds__(256, 3) k_lu_update(int k0, int nblk, int nmax, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
+                                                   double* __restrict__ A, const int32_t* __restrict__ piv, const int64_t* __restrict__ pivoff) {
+  __shared__ double sU[LU_NB][LU_COLS + 1], sL[LU_NB][LU_NB];
+  __shared__ int s_src[LU_NB], s_dst[LU_NB];
+  __shared__ unsigned s_zero;
+  const int b = blockIdx.y;
+  if (b >= nblk) return;
+  const int n = nsz[b];
+  if (n <= 0 || n > nmax || n > LU_REG_MAXN || k0 >= n) return;
+  const int nb = n - k0 < LU_NB ? n - k0 : LU_NB, k1 = k0 + LU_NB, nleft = k0 / LU_COLS;
+  const bool right = (int)blockIdx.x >= nleft;
+  const int c0 = right ? k1 + ((int)blockIdx.x - nleft) * LU_COLS : (int)blockIdx.x * LU_COLS;
+  if (c0 >= n) return;
+  double* a = A + off[b];
+  const int32_t* pb = piv + pivoff[b] + k0;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (w == 0) {
+    // where the exchanges take each row involved: lane d < 32 follows panel row k0 + d, lane 32 + q the row of pivot q
+    const int q = lane & 31, pq = q < nb ? pb[q] - 1 : k0 + q, orig = lane < 32 ? k0 + lane : pq;
+    int loc = orig;
+#pragma unroll
+    for (int i = 0; i < LU_NB; i++) {
+      const int p = __builtin_amdgcn_readlane(pq, i), j = k0 + i;
+      loc = loc == j ? p : (loc == p ? j : loc);
+    }
+    if (lane < 32) s_dst[lane] = loc;
+    if (loc >= k0 && loc < k1) s_src[loc - k0] = orig;
+    const bool z = q < nb && a[(size_t)(k0 + q) * n + k0 + q] == 0.0;
+    const unsigned long long zm = __ballot(z);
+    if (lane == 0) s_zero = (unsigned)zm;
+  }
+  __syncthreads();
+  // exchanges: thread (column, part) moves four of the panel rows
+  const int c = c0 + (t & 31), part = t >> 5;
+  const bool in = c < n;
+  double top[4], old[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int d = 4 * part + i;
+    top[i] = in && d < nb ? a[(size_t)s_src[d] * n + c] : 0.0;
+    old[i] = in && d < nb ? a[(size_t)(k0 + d) * n + c] : 0.0;
+  }
+  const unsigned zmask = s_zero;
+  if (right)
+    for (int e = t; e < LU_NB * LU_NB; e += 256) {
+      const int i = e / LU_NB, q = e % LU_NB;
+      sL[q][i] = (q < i && !((zmask >> q) & 1u)) ? a[(size_t)(k0 + i) * n + k0 + q] : 0.0;   // column q of L11
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int d = 4 * part + i;
+    if (in && d < nb) {
+      if (s_dst[d] >= k1) a[(size_t)s_dst[d] * n + c] = old[i];
+      if (!right && s_src[d] != k0 + d) a[(size_t)(k0 + d) * n + c] = top[i];
+    }
+  }
+  if (!right) return;   // (the block is uniform in this)
+  // U12 = L11^-1 A12, four rows after the other: per element the order of getf2's steps
+#pragma unroll 1
+  for (int qb = 0; qb < LU_NB / 4; qb++) {
+    if (part == qb) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+#pragma unroll
+        for (int i = q + 1; i < 4; i++) top[i] -= sL[4 * qb + q][4 * qb + i] * top[q];
+        sU[4 * qb + q][t & 31] = top[q];
+      }
+    }
+    __syncthreads();
+    if (part > qb) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const double uq = sU[4 * qb + q][t & 31];
+#pragma unroll
+        for (int i = 0; i < 4; i++) top[i] -= sL[4 * qb + q][4 * part + i] * uq;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (in) a[(size_t)(k0 + 4 * part + i) * n + c] = top[i];
+  const int col = lane & 15, grp = lane >> 4;
+  double u[2][LU_NB / 4];
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int kk = 0; kk < LU_NB / 4; kk++) u[h][kk] = sU[4 * kk + grp][16 * h + col];
+#pragma unroll 1
+  for (int r0 = k1 + 16 * w; r0 < n; r0 += 128) {   // tile rows r0 and r0 + 64, their loads together
+    double l[2][LU_NB / 4];
+    gj_f64x4 acc[2][2];
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+#pragma unroll
+      for (int kk = 0; kk < LU_NB / 4; kk++) {
+        const int q = 4 * kk + grp, r = r0 + 64 * g + col;
+        l[g][kk] = r < n && !((zmask >> q) & 1u) ? -a[(size_t)r * n + k0 + q] : 0.0;
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int r = r0 + 64 * g + grp + 4 * i, cc = c0 + 16 * h + col;
+          acc[g][h][i] = r < n && cc < n ? a[(size_t)r * n + cc] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int kk = 0; kk < LU_NB / 4; kk++)
+#pragma unroll
+      for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) acc[g][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(l[g][kk], u[h][kk], acc[g][h], 0, 0, 0);
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int r = r0 + 64 * g + grp + 4 * i, cc = c0 + 16 * h + col;
+          if (r < n && cc < n) a[(size_t)r * n + cc] = acc[g][h][i];
+        }
+  }
+}
+
+// INFO of the factored blocks: the first zero on the diagonal (1-based), 0, or -1 for an invalid size.
+__global__ void __launch_bounds__(64) k_lu_first_zero(int nblk, int nmax, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
+                                                      const double* __restrict__ A, int32_t* __restrict__ info) {
+  const int b = blockIdx.x;
+  if (b >= nblk) return;
+  const int n = nsz[b];
+  int inf = n <= 0 || n > nmax ? -1 : 0;
+  for (int j0 = 0; j0 < n && !inf; j0 += 64) {
+    const int j = j0 + (int)threadIdx.x;
+    const unsigned long long z = __ballot(j < n && A[off[b] + (int64_t)j * n + j] == 0.0);
+    if (z) inf = j0 + __builtin_ctzll(z) + 1;
+  }
+  if (threadIdx.x == 0) info[b] = inf;
+}
+
+// x_b <- LU_b \ x_b   (getrs with the 1-based pivots), two kernels that each take their block sizes.
+//
+// Up to SOLVE_SMALL DOF: one wavefront per block, lane l holds x_l and x_64+l in registers.  The
+// substitutions run column by column; the finished x_j reaches the other lanes as a scalar and the
+// factor's columns, which do not depend on it, are loaded ahead.  The forward sweep adds the terms of a
+// row in getrs' order (k = 0 .. i-1), the backward sweep from the last column.
+//
+// Above: one workgroup per block, x in LDS, SOLVE_T columns at a time: one wavefront solves the diagonal
+// tile, staged in LDS, then every wavefront subtracts the finished entries from groups of 64 rows, lane
+// by lane in the same order.  The factor does not depend on x, so the next tile and every wavefront's
+// first group are loaded (coalesced, turned in LDS) while the diagonal tile is solved.
+//
+// Bound: the 2 n dependent steps of the diagonal tiles, half of them with a division.  48 blocks of
+// 200..540 DOF: 1.67 ms by one wavefront per block walking the factor's columns in memory, 0.20 ms here;
+// 300 of 100 DOF 0.14 -> 0.08 ms.  Measured and not kept: lane partial sums of the rows (0.20 ms too, and
+// other rounding), the division by a Newton step on a reciprocal (0.23 ms).
+constexpr int SOLVE_SMALL = 128, SOLVE_T = 64, SOLVE_WAVES = 8;
+
+__global__ void __launch_bounds__(64) k_block_solve(int nblk, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
+                                                    const double* __restrict__ LU, const int32_t* __restrict__ ipiv,
+                                                    const int64_t* __restrict__ pivoff, const int64_t* __restrict__ xoff,
+                                                    double* __restrict__ x) {
+  const int b = blockIdx.x;
+  if (b >= nblk) return;
+  const int n = nsz[b];
+  if (n <= 0 || n > SOLVE_SMALL) return;
   const int lane = threadIdx.x;
-  const Real* L = LU + off[b];
+  const double* L = LU + off[b];
   const int32_t* pv = ipiv + pivoff[b];
-  Real* xb = x + xoff[b];
-  if (lane == 0)
-    for (int j = 0; j < n; j++) {
-      const int p = pv[j] - 1;
-      if (p != j) { const Real t = xb[j]; xb[j] = xb[p]; xb[p] = t; }
-    }
-  __syncthreads();   // the interchanged entries are read by their owners below
-  for (int j = 0; j < n; j++) {
-    Real xj = lane == (j & 63) ? xb[j] : Real(0);
-    xj = __shfl(xj, j & 63, 64);
-    int i = lane;
-    if (i <= j) i += ((j - lane) / 64 + 1) * 64;   // first owned row below j
-    for (; i < n; i += 64) xb[i] -= L[(size_t)i * n + j] * xj;
+  double* xb = x + xoff[b];
+  const int r[2] = {lane, lane + 64};
+  double v[2];
+  int p[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    v[h] = r[h] < n ? xb[r[h]] : 0.0;
+    p[h] = r[h] < n ? pv[r[h]] - 1 : r[h];
   }
-  for (int j = n - 1; j >= 0; j--) {
-    Real xj = Real(0);
-    if (lane == (j & 63)) {
-      xj = xb[j] / L[(size_t)j * n + j];
-      xb[j] = xj;
+  auto entry = [&](int j) { return j < 64 ? wave_read(v[0], j) : wave_read(v[1], j - 64); };   // j: uniform
+  auto set = [&](int j, double y) {
+    if (lane == (j & 63)) { if (j < 64) v[0] = y; else v[1] = y; }
+  };
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+    for (unsigned long long m = __ballot(p[h] != r[h]); m; m &= m - 1) {   // exchanges, in order
+      const int j = 64 * h + __builtin_ctzll(m), q = __builtin_amdgcn_readlane(p[h], j & 63);
+      const double xj = entry(j), xq = entry(q);
+      set(j, xq);
+      set(q, xj);
     }
-    xj = __shfl(xj, j & 63, 64);
-    for (int i = lane; i < j; i += 64) xb[i] -= L[(size_t)i * n + j] * xj;
+  // columns in batches whose loads are issued together (rows and columns clamped into the block)
+  constexpr int B = 8;
+  const double* row[2] = {L + (size_t)(r[0] < n ? r[0] : n - 1) * n, L + (size_t)(r[1] < n ? r[1] : n - 1) * n};
+  const bool two = n > 64;
+  for (int j0 = 0; j0 < n; j0 += B) {
+    double l[2][B];
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      const int j = j0 + i < n ? j0 + i : n - 1;
+      l[0][i] = row[0][j];
+      if (two) l[1][i] = row[1][j];
+    }
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      const int j = j0 + i;
+      if (j < n) {
+        const double xj = entry(j);
+        if (r[0] > j) v[0] -= l[0][i] * xj;
+        if (two && r[1] > j) v[1] -= l[1][i] * xj;
+      }
+    }
   }
+  for (int j0 = n - 1; j0 >= 0; j0 -= B) {
+    double u[2][B];
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      const int j = j0 - i > 0 ? j0 - i : 0;
+      u[0][i] = row[0][j];
+      u[1][i] = two ? row[1][j] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      const int j = j0 - i;
+      if (j >= 0) {
+        const double xj = entry(j) / (j < 64 ? wave_read(u[0][i], j) : wave_read(u[1][i], j - 64));
+        set(j, xj);
+        if (r[0] < j) v[0] -= u[0][i] * xj;
+        if (two && r[1] < j) v[1] -= u[1][i] * xj;
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+    if (r[h] < n) xb[r[h]] = v[h];
+}
+
+__global__ void __launch_bounds__(64 * SOLVE_WAVES) k_block_solve_wide(int nblk, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
+                                                                       const double* __restrict__ LU, const int32_t* __restrict__ ipiv,
+                                                                       const int64_t* __restrict__ pivoff, const int64_t* __restrict__ xoff,
+                                                                       double* __restrict__ x) {
+  constexpr int NT = 64 * SOLVE_WAVES, TE = SOLVE_T * SOLVE_T / NT;
+  __shared__ double xs[LU_BIG_MAXN];
+  __shared__ double tile[SOLVE_T][SOLVE_T + 1];
+  __shared__ double turn[SOLVE_WAVES][64][17];
+  const int b = blockIdx.x;
+  if (b >= nblk) return;
+  const int n = nsz[b];
+  if (n <= SOLVE_SMALL || n > LU_BIG_MAXN) return;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const double* L = LU + off[b];
+  const int32_t* pv = ipiv + pivoff[b];
+  double* xb = x + xoff[b];
+  for (int i = t; i < n; i += NT) xs[i] = xb[i];
+  double next[TE];        // this thread's entries of the next diagonal tile
+  auto load_tile = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < TE; i++) {
+      const int e = t + NT * i, r = k0 + e / SOLVE_T, c = k0 + e % SOLVE_T;
+      next[i] = r < n && c < n ? L[(size_t)r * n + c] : 0.0;
+    }
+  };
+  load_tile(0);
+  __syncthreads();
+  if (w == 0)
+    for (int j0 = 0; j0 < n; j0 += 64) {   // exchanges, in order; rows that stay are skipped
+      const int p = j0 + lane < n ? pv[j0 + lane] - 1 : j0 + lane;
+      for (unsigned long long m = __ballot(p != j0 + lane); m; m &= m - 1) {
+        const int i = __builtin_ctzll(m), q = __builtin_amdgcn_readlane(p, i);
+        if (lane == 0) { const double y = xs[j0 + i]; xs[j0 + i] = xs[q]; xs[q] = y; }
+      }
+    }
+  const int T = (n + SOLVE_T - 1) / SOLVE_T;
+#pragma unroll 1
+  for (int step = 0; step < 2 * T; step++) {
+    const bool lower = step < T;
+    const int k0 = SOLVE_T * (lower ? step : 2 * T - 1 - step), k1 = k0 + SOLVE_T < n ? k0 + SOLVE_T : n, m = k1 - k0;
+    const int ra = lower ? k1 : 0, rb = lower ? n : k0;   // rows the finished entries are subtracted from
+    // (the last reader of the tile, the solve below, is a barrier behind)
+#pragma unroll
+    for (int i = 0; i < TE; i++) {
+      const int e = t + NT * i;
+      tile[e / SOLVE_T][e % SOLVE_T] = next[i];
+    }
+    // columns k0 .. k1 of rows base .. base + 63, four rows of 16 columns per load
+    double pre[4][16];
+    auto load_rows = [&](int base) {
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          const int r = base + 4 * i + (lane >> 4), c = k0 + 16 * s + (lane & 15);
+          pre[s][i] = r < rb && c < k1 ? L[(size_t)r * n + c] : 0.0;
+        }
+    };
+    if (ra + 64 * w < rb) load_rows(ra + 64 * w);
+    if (step + 1 < 2 * T) load_tile(SOLVE_T * (step + 1 < T ? step + 1 : 2 * T - 2 - step));
+    __syncthreads();
+    if (w == 0) {
+      double v = lane < m ? xs[k0 + lane] : 0.0;
+      if (lower) {
+#pragma unroll 8
+        for (int j = 0; j < m; j++) {
+          const double l = tile[lane][j], xj = wave_read(v, j);
+          if (lane > j) v -= l * xj;
+        }
+      } else {
+        const double d = tile[lane][lane];
+#pragma unroll 8
+        for (int j = m - 1; j >= 0; j--) {
+          const double u = tile[lane][j];
+          if (lane == j) v = v / d;
+          const double xj = wave_read(v, j);
+          if (lane < j) v -= u * xj;
+        }
+      }
+      if (lane < m) xs[k0 + lane] = v;
+    }
+    __syncthreads();
+    for (int base = ra + 64 * w; base < rb; base += NT) {
+      if (base != ra + 64 * w) load_rows(base);
+      const int r = base + lane;
+      double y = r < rb ? xs[r] : 0.0;
+      double (*T2)[17] = turn[w];
+#pragma unroll
+      for (int ss = 0; ss < 4; ss++) {
+        auto part = [&](const double (&p)[16], int s) {
+#pragma unroll
+          for (int i = 0; i < 16; i++) T2[4 * i + (lane >> 4)][lane & 15] = p[i];
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int q = 0; q < 16; q++) {
+            const int j = lower ? q : 15 - q;
+            if (16 * s + j < m) y -= T2[lane][j] * xs[k0 + 16 * s + j];
+          }
+          __builtin_amdgcn_wave_barrier();
+        };
+        if (lower) part(pre[ss], ss);
+        else part(pre[3 - ss], 3 - ss);
+      }
+      if (r < rb) xs[r] = y;
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < n; i += NT) xb[i] = xs[i];
 }
 
 // y_b <- alpha * Ainv_b x_b + beta * y_b   (block-diagonal apply with explicit inverses, one wave per block)
@@ -1059,6 +1516,21 @@ static int lu_launch_reg(int nblk, int nmax, const int32_t* n, const int64_t* of
   return BOSSS_OK;
 }
 
+// Blocks of 129..LU_REG_MAXN DOF, panels in registers; piv: the caller's pivots.
+static int lu_launch_panels(int nblk, int nmax, const int32_t* n, const int64_t* off, double* A, int32_t* piv, const int64_t* pivoff,
+                            int32_t* info, hipStream_t s) {
+  for (int k0 = 0; k0 < nmax; k0 += LU_NB) {
+    if (nmax - k0 <= 512) hipLaunchKernelGGL(k_lu_panel_reg<256>, dim3(nblk), dim3(256), 0, s, k0, nblk, nmax, n, off, A, piv, pivoff);
+    else hipLaunchKernelGGL(k_lu_panel_reg<512>, dim3(nblk), dim3(512), 0, s, k0, nblk, nmax, n, off, A, piv, pivoff);
+    const int chunks = k0 / LU_COLS + (std::max(0, nmax - k0 - LU_NB) + LU_COLS - 1) / LU_COLS;
+    if (chunks) hipLaunchKernelGGL(k_lu_update, dim3(chunks, nblk), dim3(256), 0, s, k0, nblk, nmax, n, off, A, piv, pivoff);
+  }
+  if (info) hipLaunchKernelGGL(k_lu_first_zero, dim3(nblk), dim3(64), 0, s, nblk, nmax, n, off, A, info);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { g_lu_err = hipGetErrorString(e); return BOSSS_ERR_HIP; }
+  return BOSSS_OK;
+}
+
 // The split form (two launches per panel) with its per-block status words st[2 nblk] in device
 // memory the caller provides; queued on s, not synchronised.
 static hipError_t lu_launch_split(int nblk, int nmax, const int32_t* n, const int64_t* off, double* A, int32_t* ipiv,
@@ -1084,6 +1556,9 @@ int bosss_hip_block_lu_dev(bosss_ctx* ctx, int nblk, int32_t nmax, const int32_t
   if (nmax <= LU_MAXN) return lu_launch_reg(nblk, nmax, n, off, A, ipiv, pivoff, info, want_inverse, (hipStream_t)stream);
   if (want_inverse) { g_lu_err = "inverses are limited to blocks of 128 DOF"; return BOSSS_ERR_UNSUPPORTED; }
   hipStream_t s = (hipStream_t)stream;
+  // Panels in registers up to LU_REG_MAXN DOF (two rows a thread).  They keep no state but the pivots, so a
+  // call without ipiv takes the forms below, as larger blocks do; a grid's y extent bounds the batch.
+  if (nmax <= LU_REG_MAXN && ipiv && nblk <= 65535) return lu_launch_panels(nblk, nmax, n, off, A, ipiv, pivoff, info, s);
   if (nmax >= LU_SPLIT_MINN && nblk < LU_SPLIT_MAXBLK) {
     // few large blocks: two launches per panel, the trailing update over many workgroups
     int32_t* st = nullptr;
@@ -1112,6 +1587,7 @@ int bosss_hip_block_lu_noalloc_dev(bosss_ctx* ctx, int nblk, int32_t nmax, const
                " DOF exceed its scratch (at most " + std::to_string(LU_NOALLOC_MAXBLK) + " per call)";
     return BOSSS_ERR_ARG;
   }
+  if (nmax <= LU_REG_MAXN && ipiv) return lu_launch_panels(nblk, nmax, n, off, A, ipiv, pivoff, info, (hipStream_t)stream);
   int32_t* st = nullptr;
   if (int rc = scratch_on_current_device(&st)) return rc;
   hipError_t e = lu_launch_split(nblk, nmax, n, off, A, ipiv, pivoff, info, st, (hipStream_t)stream);
@@ -1124,8 +1600,8 @@ int bosss_hip_block_solve_dev(bosss_ctx* ctx, int nblk, const int32_t* n, const 
   if (nblk <= 0) return BOSSS_OK;
   if (int rc = select_device(ctx)) return rc;
   if (!n || !off || !LU || !ipiv || !pivoff || !xoff || !x) { g_lu_err = "NULL argument"; return BOSSS_ERR_ARG; }
-  hipLaunchKernelGGL(k_block_solve<double>, dim3(nblk), dim3(64), 0, (hipStream_t)stream, nblk, n, off, LU, ipiv,
-                     pivoff, xoff, x);
+  hipLaunchKernelGGL(k_block_solve, dim3(nblk), dim3(64), 0, (hipStream_t)stream, nblk, n, off, LU, ipiv, pivoff, xoff, x);
+  hipLaunchKernelGGL(k_block_solve_wide, dim3(nblk), dim3(64 * SOLVE_WAVES), 0, (hipStream_t)stream, nblk, n, off, LU, ipiv, pivoff, xoff, x);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { g_lu_err = hipGetErrorString(e); return BOSSS_ERR_HIP; }
   return BOSSS_OK;
