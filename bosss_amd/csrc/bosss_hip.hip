@@ -83,6 +83,7 @@ struct bosss_op {
   void* tables;      // packed tables (Real) on the device
   void* ttab;        // 1D tensor tables (Real) on the device, if the uploaded tables are a tensor product
   bool tensor;
+  bool split[KernelSet::NVARIANT] = {false, false, false, false};   // cell-split kernels (split_pays)
   FormParams fp;
   size_t ndof;
   // staging buffers for the host-pointer entry points
@@ -435,6 +436,23 @@ static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks,
   return md <= 1e-12 * scale;
 }
 
+// Whether the cell-split form of a kernel is taken.  A CU works through w = ceil(J / 64 / CUs) groups
+// of 64 cells or w4 = ceil(J / 16 / CUs) groups of 16, and a group of 16 takes `turn` of a group of 64:
+// a quarter and what a workgroup does once whatever its cells (tables into LDS, metrics, the sum of
+// the parts), which weighs more the less there is to do.  HLLC, us without / with the split form:
+//   p = 3 JVP       5^3 171 / 53, 20^3 182 / 117, 25^3 195 / 228, 31 x 29 x 37 548 / 491, 48^3 1260 / 1440
+//   p = 3 fused     5^3 227 / 70, 20^3 240 / 155, 25^3 256 / 300, 31 x 29 x 37 712 / 644, 48^3 1632 / 1888
+//   p = 3 residual  5^3 101 / 36, 20^3 108 /  77, 25^3 118 / 150, 31 x 29 x 37 335 / 331, 48^3  775 / 1033
+//   p = 2 JVP       5^3  69 / 27, 20^3  75 /  58, 25^3  82 / 111, 31 x 29 x 37 228 / 242, 48^3  537 /  709
+// BOSSS_HIP_SPLIT=0 or 1 decides instead.
+static bool split_pays(int J, int num_cu, int D, int P, bool residual) {
+  if (const char* x = std::getenv("BOSSS_HIP_SPLIT")) return x[0] == '1';
+  // 2D: one volume tile, so a group of 16 takes more than half of a group of 64 (fused 80 x 80: 22 / 25 us)
+  const double turn = D == 2 ? 0.51 : P == 3 ? (residual ? 0.325 : 0.31) : 0.345;
+  const int w = ((J + 16 * TWAVES - 1) / (16 * TWAVES) + num_cu - 1) / num_cu, w4 = ((J + 15) / 16 + num_cu - 1) / num_cu;
+  return turn * w4 < w;
+}
+
 extern "C" {
 
 int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tables_desc* t, int kind,
@@ -504,6 +522,11 @@ int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tabl
     add(t->face_weights, Ke); add(t->trace, NF * Ke * N); add(t->dtrace, NF * Ke * N * D);
   }
   if ((rc = ks->prepare()) != 0) { bosss_hip_op_destroy(op); return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc); }
+  if (op->tensor)
+    for (int i = 0; i < KernelSet::NVARIANT; i++) {
+      const void* part = precision == BOSSS_FP64 ? (const void*)ks->kts64[i] : (const void*)ks->kts32[i];
+      if (part) op->split[i] = split_pays(grid->J, ctx->num_cu, t->D, ks->P, i == KernelSet::RES);
+    }
   *out = op;
   return BOSSS_OK;
 }
@@ -603,7 +626,9 @@ static int launch(bosss_op* op, int which, double alpha, double beta, const void
     if (op->ks->km32[which]) return launch_modal<float>(op, op->ks->km32[which], alpha, beta, U, X, R, out, s);
   }
   if (op->tensor) {
-    dim3 grid((op->grid->J + 16 * TWAVES - 1) / (16 * TWAVES)), block(64 * TWAVES);
+    const bool split = op->split[which];
+    const int cells = split ? 16 : 16 * TWAVES;   // per workgroup
+    dim3 grid((op->grid->J + cells - 1) / cells), block(64 * TWAVES);
     // Plane-fastest workgroup order (xcd_block) for the Euler JVP and VJP kernels when one
     // plane's operands (U and the tangent or cotangent) exceed half of an XCD's 4 MB L2: in the
     // range order they are evicted before the next plane's workgroups re-read them (64^3, p = 3:
@@ -611,16 +636,16 @@ static int launch(bosss_op* op, int which, double alpha, double beta, const void
     // with it and keeps the range order, as do smaller planes, whose re-reads already hit L2.
     const bool euler = op->kind == BOSSS_FORM_EULER_LF || op->kind == BOSSS_FORM_EULER_HLLC;
     const size_t plane_bytes = (size_t)op->grid->plane * 2 * op->V * op->N * (op->precision == BOSSS_FP64 ? 8 : 4);
-    const int plane_blocks = (euler && which != KernelSet::RES && op->grid->plane % (16 * TWAVES) == 0 &&
+    const int plane_blocks = (euler && which != KernelSet::RES && op->grid->plane % cells == 0 &&
                               plane_bytes > (size_t(2) << 20))
-                                 ? op->grid->plane / (16 * TWAVES) : 0;
+                                 ? op->grid->plane / cells : 0;
     if (op->precision == BOSSS_FP64) {
-      void (*k)(TArgs<double>) = op->ks->kt64[which];
+      void (*k)(TArgs<double>) = split ? op->ks->kts64[which] : op->ks->kt64[which];
       if (!k) return fail(BOSSS_ERR_UNSUPPORTED, "tensor kernel variant %d not built", which);
       hipLaunchKernelGGL(k, grid, block, op->ks->ktlds64[which], s,
                          make_targs<double>(op, alpha, beta, U, X, R, out, own_only, plane_blocks));
     } else {
-      void (*k)(TArgs<float>) = op->ks->kt32[which];
+      void (*k)(TArgs<float>) = split ? op->ks->kts32[which] : op->ks->kt32[which];
       if (!k) return fail(BOSSS_ERR_UNSUPPORTED, "tensor kernel variant %d not built", which);
       hipLaunchKernelGGL(k, grid, block, op->ks->ktlds32[which], s,
                          make_targs<float>(op, alpha, beta, U, X, R, out, own_only, plane_blocks));

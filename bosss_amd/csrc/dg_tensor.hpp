@@ -320,6 +320,42 @@ template <int D> struct IsHLLC<FormEuler<D, true>> : std::true_type {};
 
 constexpr int TWAVES = 4;
 
+// Cell-split form of the Euler kernels (SPLIT): the TWAVES wavefronts of a workgroup share one group
+// of 16 cells instead of taking one each.  Wavefront w takes the volume tiles w, w + TWAVES, ... and
+// a contiguous share of the face tiles (all faces of the cell, TE tiles each), and the partial results
+// are added through LDS in wavefront order.  The work unit is a quarter as long, for grids whose groups of
+// 64 cells leave CUs idle (split_pays).
+template <class TS>
+struct FaceShare {
+  int lo, hi;   // face tiles f * TE + t of this wavefront
+  __device__ __forceinline__ FaceShare(bool split, int wave)
+      : lo(split ? wave * TS::NF * TS::TE / TWAVES : 0), hi(split ? (wave + 1) * TS::NF * TS::TE / TWAVES : TS::NF * TS::TE) {}
+  __device__ __forceinline__ int f0() const { return lo / TS::TE; }
+  __device__ __forceinline__ int f1() const { return (hi + TS::TE - 1) / TS::TE; }
+  __device__ __forceinline__ int t0(int f) const { return lo > f * TS::TE ? lo - f * TS::TE : 0; }
+  __device__ __forceinline__ int t1(int f) const { return hi < (f + 1) * TS::TE ? hi - f * TS::TE : TS::TE; }
+};
+
+// This wavefront's accumulators to part[c * (NT | 1) + i] (cell c, entry i).
+template <class TS, typename Real, int V>
+__device__ __forceinline__ void split_put(Real* part, int col, int grp, const TAcc<TS, Real, V>& acc) {
+  constexpr int STRIDE = (V * TS::N) | 1;
+  acc.store(grp, [&](int v, int n, Real val) { part[col * STRIDE + v * TS::N + n] = val; });
+}
+// out <- be out + al (sum of the wavefronts' parts, `step` apart), the workgroup's 16 cells in whole lines.
+template <typename Real, int NT>
+__device__ __forceinline__ void split_sum(const Real* part, int step, Real* __restrict__ out, int cell0, int J, Real al, Real be) {
+  for (int i = threadIdx.x; i < 16 * NT; i += 64 * TWAVES) {
+    const int c = i / NT, e = i - c * NT;
+    if (cell0 + c >= J) break;
+    Real s = part[c * (NT | 1) + e];
+#pragma unroll
+    for (int w = 1; w < TWAVES; w++) s += part[w * step + c * (NT | 1) + e];
+    Real* o = out + (size_t)cell0 * NT + i;
+    *o = be != Real(0) ? be * *o + al * s : al * s;
+  }
+}
+
 // Face tables kt_forward and kt_adjoint load: the trace table, and for forms whose faces use
 // gradients (SIP, advection-diffusion) the D reference-derivative tables as well.
 template <class Form, int D>
@@ -339,7 +375,7 @@ constexpr int adjoint_min_waves() { return (sizeof(Real) == 4 || (P < 3 && !FUSE
 // ----------------------------------------------------------------------------
 // Forward: residual (MODE_RES) or JVP (MODE_JVP).
 // ----------------------------------------------------------------------------
-template <class Form, int D, int P, int K1, typename Real, int MODE>
+template <class Form, int D, int P, int K1, typename Real, int MODE, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt_forward(TArgs<Real> a) {
   typedef TShape<D, P, K1> TS;
   typedef typename MM<Real>::acc acc_t;
@@ -354,7 +390,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   for (int i = threadIdx.x; i < TS::TAB; i += blockDim.x) tab[i] = a.tab[i];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int cell0 = (xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16;
+  const int cell0 = (SPLIT ? xcd_block(a.nxcd, a.plane_blocks) : xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16;
   Real* stU = tab + ((TS::TAB + 1) & ~1) + wave * (NARR * 16 * STRIDE);
   Real* stX = stU + 16 * STRIDE;
   // face tables: traces, and the reference-derivative traces where the faces use gradients
@@ -385,7 +421,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   auto Bx = [&](int v, int kk) { int m = 4 * kk + grp; return ownX[v * N + (m < N ? m : N - 1)] * ((m < N) ? sc : Real(0)); };
 
   // ------------------------------------------------------------------ volume
-  for (int t = 0; t < TS::TV; t++) {
+  for (int t = SPLIT ? wave : 0; t < TS::TV; t += SPLIT ? TWAVES : 1) {
     int qe[3];
     const int nodeE = t * 16 + col;
     vol_axes<D, K1>(nodeE < TS::KV ? nodeE : 0, qe);
@@ -444,7 +480,8 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   // ------------------------------------------------------------------- faces
   const Real pbd = Real(a.fp.penalty_base * a.fp.penalty_deg);
   const Real cj_own = Real(1.0 / a.lenscale[cj]);
-  for (int f = 0; f < NF; f++) {
+  const FaceShare<TS> share(SPLIT, wave);
+  for (int f = share.f0(); f < share.f1(); f++) {
     const int nb_raw = a.cf.nb[(size_t)cj * NF + f];
     const int nb = valid ? nb_raw : -1;
     const bool has_nb = nb >= 0;
@@ -467,7 +504,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
     auto Bnu = [&](int v, int kk) { int m = 4 * kk + grp; return nbU[v * N + (m < N ? m : N - 1)] * ((has_nb && m < N) ? scn : Real(0)); };
     auto Bnx = [&](int v, int kk) { int m = 4 * kk + grp; return nbX[v * N + (m < N ? m : N - 1)] * ((has_nb && !a.own_only && m < N) ? scn : Real(0)); };
 
-    for (int t = 0; t < TS::TE; t++) {
+    for (int t = share.t0(f); t < share.t1(f); t++) {
       // trace operands FT(f, node, mode) and FT(fo, node, mode) of the tile's nodes; the
       // derivative table of direction e follows at (1 + e) FTAB
       const Real* fto = ft + (f * TS::FROWS + t * 16 + col) * TS::FS + grp;
@@ -558,6 +595,13 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
     }
   }
 
+  if constexpr (SPLIT) {
+    split_put<TS, Real, V>(stU, col, grp, racc);   // own cells' coefficients are not read any more
+    __syncthreads();
+    split_sum<Real, NT>(tab + ((TS::TAB + 1) & ~1), NARR * 16 * STRIDE, TAN ? a.out : a.R, cell0, a.J, TAN ? Real(1) : Real(a.alpha),
+                        TAN ? Real(0) : Real(a.beta));
+    return;
+  }
   if (valid) {
     Real* Op = (TAN ? a.out : a.R) + (size_t)cell * NT;
     const Real al = Real(a.alpha), be = Real(a.beta);
@@ -937,7 +981,7 @@ namespace bosss {
 template <typename Real, int P, bool FUSED>
 constexpr int vjp_euler_min_waves() { return (sizeof(Real) == 4 && (FUSED || P < 3)) ? 2 : 1; }
 
-template <class Form, int D, int P, int K1, typename Real, bool FUSED>
+template <class Form, int D, int P, int K1, typename Real, bool FUSED, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUSED>())) kt_vjp_euler(TArgs<Real> a) {
   typedef TShape<D, P, K1> TS;
   typedef typename MM<Real>::acc acc_t;
@@ -956,7 +1000,8 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
   const FtCols<TS, Real, V> ftc(col);
   auto slot = [&](int arr, int v, int r) -> Real& { return buf[((arr * V + v) * 4 + r) * 64 + lane]; };
 
-  const int cell = (xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16 + col;
+  const int cell0 = (SPLIT ? xcd_block(a.nxcd, a.plane_blocks) : xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16;
+  const int cell = cell0 + col;
   const bool valid = cell < a.J;
   const int cj = valid ? cell : 0;
   const Real sc = Real(a.scaling[cj]);
@@ -1013,7 +1058,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
   };
 
   // ------------------------------------------------------------------ volume
-  for (int t = 0; t < TS::TV; t++) {
+  for (int t = SPLIT ? wave : 0; t < TS::TV; t += SPLIT ? TWAVES : 1) {
     int qe[3];
     const int nodeE = t * 16 + col;
     vol_axes<D, K1>(nodeE < TS::KV ? nodeE : 0, qe);
@@ -1093,7 +1138,8 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
   }
 
   // ------------------------------------------------------------------- faces
-  for (int f = 0; f < NF; f++) {
+  const FaceShare<TS> share(SPLIT, wave);
+  for (int f = share.f0(); f < share.f1(); f++) {
     const int nb_raw = a.cf.nb[(size_t)cj * NF + f];
     const int nb = valid ? nb_raw : -1;
     const bool has_nb = nb >= 0;
@@ -1108,7 +1154,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
     const Real* nbW = a.X + (size_t)cn * NT;
     auto Bnu = [&](int v, int kk) { int m = 4 * kk + grp; return nbU[v * N + (m < N ? m : N - 1)] * ((has_nb && m < N) ? scn : Real(0)); };
 
-    for (int t = 0; t < TS::TE; t++) {
+    for (int t = share.t0(f); t < share.t1(f); t++) {
       // trace operands FT(f, node, mode) and FT(fo, node, mode) of the tile's nodes
       const Real* fto = ft + (f * TS::FROWS + t * 16 + col) * TS::FS + grp;
       const Real* ftn = ft + (fo * TS::FROWS + t * 16 + col) * TS::FS + grp;
@@ -1171,6 +1217,17 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
     }
   }
 
+  if constexpr (SPLIT) {
+    constexpr int PART = 16 * (NT | 1);
+    static_assert(2 * PART <= NSLOT * 64, "both results fit the node buffer");
+    Real* parts = tab + ((TS::TAB + 1) & ~1);
+    split_put<TS, Real, V>(buf, col, grp, aacc);
+    if (FUSED) split_put<TS, Real, V>(buf + PART, col, grp, racc);
+    __syncthreads();
+    split_sum<Real, NT>(parts, NSLOT * 64, a.out, cell0, a.J, Real(1), Real(0));
+    if (FUSED) split_sum<Real, NT>(parts + PART, NSLOT * 64, a.R, cell0, a.J, Real(a.alpha), Real(a.beta));
+    return;
+  }
   if (valid) {
     Real* Rp = FUSED ? a.R + (size_t)cell * NT : nullptr;
     Real* Op = a.out + (size_t)cell * NT;
@@ -1189,7 +1246,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
 // tangent trace of a 16-node face tile are parked in LDS, the neighbour tangent
 // trace stays in registers; the dual-number flux is then evaluated node by node.
 // ----------------------------------------------------------------------------
-template <class Form, int D, int P, int K1, typename Real>
+template <class Form, int D, int P, int K1, typename Real, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 2 : 1))) kt_jvp_euler(TArgs<Real> a) {
   typedef TShape<D, P, K1> TS;
   typedef typename MM<Real>::acc acc_t;
@@ -1209,7 +1266,8 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   const FtCols<TS, Real, V> ftc(col);
   auto slot = [&](int arr, int v, int r) -> Real& { return buf[((arr * V + v) * 4 + r) * 64 + lane]; };
 
-  const int cell = (xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16 + col;
+  const int cell0 = (SPLIT ? xcd_block(a.nxcd, a.plane_blocks) : xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16;
+  const int cell = cell0 + col;
   const bool valid = cell < a.J;
   const int cj = valid ? cell : 0;
   const Real sc = Real(a.scaling[cj]);
@@ -1266,7 +1324,7 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   };
 
   // ------------------------------------------------------------------ volume
-  for (int t = 0; t < TS::TV; t++) {
+  for (int t = SPLIT ? wave : 0; t < TS::TV; t += SPLIT ? TWAVES : 1) {
     int qe[3];
     const int nodeE = t * 16 + col;
     vol_axes<D, K1>(nodeE < TS::KV ? nodeE : 0, qe);
@@ -1307,7 +1365,8 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   }
 
   // ------------------------------------------------------------------- faces
-  for (int f = 0; f < NF; f++) {
+  const FaceShare<TS> share(SPLIT, wave);
+  for (int f = share.f0(); f < share.f1(); f++) {
     const int nb_raw = a.cf.nb[(size_t)cj * NF + f];
     const int nb = valid ? nb_raw : -1;
     const bool has_nb = nb >= 0;
@@ -1323,7 +1382,7 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
     auto Bnu = [&](int v, int kk) { int m = 4 * kk + grp; return nbU[v * N + (m < N ? m : N - 1)] * ((has_nb && m < N) ? scn : Real(0)); };
     auto Bnx = [&](int v, int kk) { int m = 4 * kk + grp; return nbX[v * N + (m < N ? m : N - 1)] * ((has_nb && !a.own_only && m < N) ? scn : Real(0)); };
 
-    for (int t = 0; t < TS::TE; t++) {
+    for (int t = share.t0(f); t < share.t1(f); t++) {
       // trace operands FT(f, node, mode) and FT(fo, node, mode) of the tile's nodes
       const Real* fto = ft + (f * TS::FROWS + t * 16 + col) * TS::FS + grp;
       const Real* ftn = ft + (fo * TS::FROWS + t * 16 + col) * TS::FS + grp;
@@ -1375,6 +1434,13 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
     }
   }
 
+  if constexpr (SPLIT) {
+    static_assert(16 * (NT | 1) <= NSLOT * 64, "the result fits the node buffer");
+    split_put<TS, Real, V>(buf, col, grp, racc);
+    __syncthreads();
+    split_sum<Real, NT>(tab + ((TS::TAB + 1) & ~1), NSLOT * 64, a.out, cell0, a.J, Real(1), Real(0));
+    return;
+  }
   if (valid) {
     Real* Op = a.out + (size_t)cell * NT;
     racc.store(grp, [&](int v, int n, Real val) { Op[v * N + n] = val; });

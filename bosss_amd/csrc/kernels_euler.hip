@@ -5,8 +5,8 @@
 
 namespace bosss {
 // The 3D p = 3 tensor kernels are compiled in their own translation units: the FP64 fused
-// residual + VJP in kernels_euler_fused.hip, the others in kernels_euler_p3.hip (built in
-// parallel with this one, each with its own scheduling flags).
+// residual + VJP in kernels_euler_fused.hip, the others in kernels_euler_p3.hip, the cell-split
+// forms in kernels_euler_split.hip (built in parallel with this one, with their own scheduling flags).
 extern template __global__ void kt_vjp_euler<FormEuler<3, false>, 3, 3, 5, double, true>(TArgs<double>);
 extern template __global__ void kt_vjp_euler<FormEuler<3, true>, 3, 3, 5, double, true>(TArgs<double>);
 #define BOSSS_EULER_P3_EXTERN(H)                                                                           \
@@ -16,7 +16,15 @@ extern template __global__ void kt_vjp_euler<FormEuler<3, true>, 3, 3, 5, double
   extern template __global__ void kt_jvp_euler<FormEuler<3, H>, 3, 3, 5, float>(TArgs<float>);            \
   extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, double, false>(TArgs<double>);   \
   extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, float, false>(TArgs<float>);     \
-  extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, float, true>(TArgs<float>);
+  extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, float, true>(TArgs<float>);       \
+  extern template __global__ void kt_forward<FormEuler<3, H>, 3, 3, 5, double, MODE_RES, true>(TArgs<double>); \
+  extern template __global__ void kt_forward<FormEuler<3, H>, 3, 3, 5, float, MODE_RES, true>(TArgs<float>); \
+  extern template __global__ void kt_jvp_euler<FormEuler<3, H>, 3, 3, 5, double, true>(TArgs<double>);     \
+  extern template __global__ void kt_jvp_euler<FormEuler<3, H>, 3, 3, 5, float, true>(TArgs<float>);       \
+  extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, double, false, true>(TArgs<double>); \
+  extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, float, false, true>(TArgs<float>); \
+  extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, double, true, true>(TArgs<double>); \
+  extern template __global__ void kt_vjp_euler<FormEuler<3, H>, 3, 3, 5, float, true, true>(TArgs<float>);
 BOSSS_EULER_P3_EXTERN(false)
 BOSSS_EULER_P3_EXTERN(true)
 #undef BOSSS_EULER_P3_EXTERN

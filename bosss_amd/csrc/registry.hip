@@ -29,6 +29,8 @@ int KernelSet::prepare() const {
     if (k64[i] && hipFuncSetAttribute((const void*)k64[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64) != hipSuccess) return 1;
     if (k32[i] && hipFuncSetAttribute((const void*)k32[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds32) != hipSuccess) return 2;
     if (kt64[i] && hipFuncSetAttribute((const void*)kt64[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds64[i]) != hipSuccess) return 3;
+    if (kts64[i] && hipFuncSetAttribute((const void*)kts64[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds64[i]) != hipSuccess) return 5;
+    if (kts32[i] && hipFuncSetAttribute((const void*)kts32[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds32[i]) != hipSuccess) return 6;
     if (kt32[i] && hipFuncSetAttribute((const void*)kt32[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds32[i]) != hipSuccess) return 4;
   }
   return 0;

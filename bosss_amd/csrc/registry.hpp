@@ -24,6 +24,9 @@ struct KernelSet {
   void (*kt64[NVARIANT])(TArgs<double>);
   void (*kt32[NVARIANT])(TArgs<float>);
   size_t ktlds64[NVARIANT], ktlds32[NVARIANT];
+  // cell-split forms of the Euler kernels (same LDS), or nullptr
+  void (*kts64[NVARIANT])(TArgs<double>);
+  void (*kts32[NVARIANT])(TArgs<float>);
   // modal kernels (dg_modal.hpp) of the linear scalar forms on axis-aligned grids, or nullptr
   void (*km64[NVARIANT])(MArgs<double>);
   void (*km32[NVARIANT])(MArgs<float>);
@@ -56,6 +59,16 @@ void set_tensor_linearisations(void (**kt)(TArgs<Real>), size_t* lds) {
   }
 }
 
+template <class Form, int D, int P, int K1, typename Real>
+void set_split(void (**kt)(TArgs<Real>)) {
+  if constexpr (HandAdjoint<Form>::value) {
+    kt[KernelSet::RES] = kt_forward<Form, D, P, K1, Real, MODE_RES, true>;
+    kt[KernelSet::JVP] = kt_jvp_euler<Form, D, P, K1, Real, true>;
+    kt[KernelSet::VJP] = kt_vjp_euler<Form, D, P, K1, Real, false, true>;
+    kt[KernelSet::RES_VJP] = kt_vjp_euler<Form, D, P, K1, Real, true, true>;
+  }
+}
+
 template <class Form> struct ModalForm : std::false_type {};
 template <> struct ModalForm<FormSIP> : std::true_type {};
 template <> struct ModalForm<FormAdvDiff> : std::true_type {};
@@ -85,7 +98,7 @@ KernelSet make_kernel_set(int kind) {
   k.k64[KernelSet::RES_VJP] = k_adjoint<Form, D, N, K1, double, true>;
   for (int i = 0; i < KernelSet::NVARIANT; i++) {
     k.k32[i] = nullptr; k.kt32[i] = nullptr; k.ktlds32[i] = 0;
-    k.km64[i] = nullptr; k.km32[i] = nullptr;
+    k.km64[i] = nullptr; k.km32[i] = nullptr; k.kts64[i] = nullptr; k.kts32[i] = nullptr;
   }
   constexpr int P = degree_from_modes(D, N);
   static_assert(tdeg_count(D, P) == N, "N must be a full total-degree basis");
@@ -96,6 +109,7 @@ KernelSet make_kernel_set(int kind) {
   k.kt64[KernelSet::RES] = kt_forward<Form, D, P, K1, double, MODE_RES>;
   k.ktlds64[KernelSet::RES] = kt_forward_lds_bytes<Form, D, P, K1, double>(1);
   set_tensor_linearisations<Form, D, P, K1, double>(k.kt64, k.ktlds64);
+  set_split<Form, D, P, K1, double>(k.kts64);
   if constexpr (ModalForm<Form>::value) {
     static_assert(K1 >= P + 1, "the modal kernels replace a rule that is exact for products of two modes");
     set_modal<Form, D, P, double>(k.km64);
@@ -105,6 +119,7 @@ KernelSet make_kernel_set(int kind) {
     k.kt32[KernelSet::RES] = kt_forward<Form, D, P, K1, float, MODE_RES>;
     k.ktlds32[KernelSet::RES] = kt_forward_lds_bytes<Form, D, P, K1, float>(1);
     set_tensor_linearisations<Form, D, P, K1, float>(k.kt32, k.ktlds32);
+    set_split<Form, D, P, K1, float>(k.kts32);
     k.k32[KernelSet::RES] = k_forward<Form, D, N, K1, float, MODE_RES>;
     k.k32[KernelSet::JVP] = k_forward<Form, D, N, K1, float, MODE_JVP>;
     k.k32[KernelSet::VJP] = k_adjoint<Form, D, N, K1, float, false>;
