@@ -361,7 +361,8 @@ static void legendre_normalised(int P, double x, double* L, double* DL) {
 static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks, int K1, std::vector<double>& tab, double* maxdiff) {
   const int D = t->D, P = ks->P, K2 = ks->t_k2, N = t->N;
   tab.assign(ks->ttab_size, 0.0);
-  if (t->Ke > ks->t_frows || ks->t_ftab != 2 * D * ks->t_frows * ks->t_fs || ks->t_o_ft + (1 + D) * ks->t_ftab != ks->ttab_size)
+  if (t->Ke > ks->t_frows || ks->t_ftab != 2 * D * ks->t_frows * ks->t_fs || ks->t_o_ft + (1 + D) * ks->t_ftab != ks->t_o_vt ||
+      ks->t_o_vt + ks->t_vrows * ks->t_fs != ks->ttab_size || t->Kv > ks->t_vrows)
     return false;
   std::vector<double> x, w;
   gauss_legendre(K1, x, w);
@@ -404,6 +405,35 @@ static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks,
       cmp(val(q, ex[n], -1), t->phi[k * N + n]);
       for (int d = 0; d < D; d++) cmp(val(q, ex[n], d), t->dphi[(k * N + n) * D + d]);
     }
+  }
+  // derivative terms: ratios of the tables' values in the upper corner, a = num / den as hi + lo
+  for (int n = 0; n < N; n++) {
+    double* dt = &tab[ks->t_o_dt + (size_t)n * 3 * (D + 1)];
+    const int up[3] = {K1 + 1, K1 + 1, K1 + 1};
+    auto ratio = [&](int slot, int index, double num, double den) {
+      const double hi = num / den;
+      dt[slot] = index;
+      dt[D + 1 + slot] = hi;
+      dt[2 * (D + 1) + slot] = std::fma(-hi, den, num) / den;
+    };
+    for (int e = 0; e < D; e++) {
+      const int a = (ex[n] >> (4 * e)) & 15;
+      if (a < 1) continue;   // slot 0, coefficient 0
+      const int i = (int)(std::find(ex.begin(), ex.end(), ex[n] - (1 << (4 * e))) - ex.begin());
+      if (i >= ks->t_np) return false;
+      if (a < 3) {
+        ratio(e, e * ks->t_np + i, val(up, ex[n], e), val(up, ex[i], -1));
+      } else {               // a pure cubic: its share of phi_0 integrates to the difference of its traces
+        ratio(D, e * ks->t_np, val(up, ex[n], -1), val(up, ex[0], -1));
+        ratio(e, e * ks->t_np + i, val(up, ex[n], e) - val(up, ex[n], -1), val(up, ex[i], -1));
+      }
+    }
+  }
+  for (int k = 0; k < ks->t_vrows; k++) {   // volume table; the padding rows repeat node 0
+    const int kn = k < t->Kv ? k : 0;
+    int q[3] = {kn % K1, (kn / K1) % K1, kn / (K1 * K1)};
+    if (D == 2) q[2] = 0;
+    for (int n = 0; n < N; n++) tab[ks->t_o_vt + (size_t)k * ks->t_fs + n] = val(q, ex[n], -1);
   }
   for (int f = 0; f < 2 * D; f++)
     for (int k = 0; k < t->Ke; k++) {

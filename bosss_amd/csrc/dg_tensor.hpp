@@ -49,7 +49,12 @@ struct TShape {
   static constexpr int TV = (KV + 15) / 16, TE = (KE + 15) / 16;
   static constexpr int NK = (N + 3) / 4, MT = (N + 15) / 16;
   static constexpr int O_L = 0, O_DL = (P + 1) * K2, O_W = 2 * (P + 1) * K2, O_CODE = O_W + K1;
-  static constexpr int TAB = O_CODE + N;     // elements (Real) of the 1D table block
+  // Derivative terms of mode m at O_DT + m * DT: d phi_m / d xi_e = c_e phi_(i_e) (+ c_3 phi_0 along the
+  // axis of a pure cubic): D + 1 slots (e * NP + i_e, the cubic's last), their coefficients, and what
+  // rounding took from these.  All modes i are of degree < P, the first NP.
+  static constexpr int NP = tdeg_count(D, P - 1), DT = 3 * (D + 1), O_DT = O_CODE + N;
+  static_assert(P <= 3, "one second derivative term per mode");
+  static constexpr int TAB = O_DT + N * DT;  // elements (Real) of the 1D table block
   // Face trace table FT[f][node][m] = phi_m at node `node` of face f, stored after the 1D block
   // in global memory: FROWS rows per face (whole 16-node tiles; the padding rows node >= KE hold
   // node 0's values, so a trace evaluated at them is a valid state), FS Real per row (modes
@@ -59,6 +64,9 @@ struct TShape {
   static constexpr int FTAB = NF * FROWS * FS;
   // 1 + D face tables in this layout follow each other: phi_m, then d phi_m / d xi_e, e < D.
   static constexpr int NFTAB = 1 + D;
+  // Volume table phi_m at the volume nodes, rows and padding as in the face tables, after them.
+  static constexpr int VTAB = TV * 16 * FS, O_VT = TAB + NFTAB * FTAB;
+  static_assert(VTAB <= FTAB, "the JVP and VJP kernels keep the volume table where the face table goes later");
 };
 
 // Per-axis 1D indices of a node: volume node kv = (i*K1 + j)*K1 + k has x = k, y = j, z = i
@@ -159,6 +167,18 @@ struct TAcc {
       rem[REM ? v : 0] = Real(0);
     }
   }
+  // t[v][n] += f(n) for every coefficient row n < N this lane holds
+  template <class F>
+  __device__ __forceinline__ void add(int v, int grp, F f) {
+#pragma unroll
+    for (int mt = 0; mt < MF; mt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        int n = mt * 16 + MM<Real>::row(grp, r);
+        if (n < TS::N) t[v][mt][r] += f(n);
+      }
+    if (REM) rem[REM ? v : 0] += f(MF * 16 + grp);
+  }
   // f(v, n, value) for every coefficient row n < N this lane holds
   template <class F>
   __device__ __forceinline__ void store(int grp, F f) const {
@@ -250,6 +270,89 @@ __device__ __forceinline__ void t_test_ft(const Real* nrow, const FtCols<TS, Rea
 }
 
 template <class TS, typename Real>
+__device__ __forceinline__ void vt_load(Real* vt, const Real* gtab) {
+  for (int i = threadIdx.x; i < TS::VTAB; i += blockDim.x) vt[i] = gtab[TS::O_VT + i];
+}
+
+// Volume test of the Euler forms, sum_e sum_k d_e phi_m g_e, by projection: d_e phi_m is a combination of
+// the NP modes of degree < P, so the nodes are contracted with those alone,
+//     Q_e,n = sum_k phi_n(k) g_e(k)       (n < NP: 10 of 20 modes at p = 3, 4 of 10 at p = 2),
+// and R_m = sum_e D_e[m][n] Q_e,n once per cell (q_fold).  A constant flux has to cancel between volume
+// and faces: D is the ratio of the rounded tables, with its own rounding error beside it (without: p = 2
+// residuals up to 24 % further from 64-bit exact).  The three directions share one operand, a
+// volume-table read, where the derivative tables took three 1D factors and a mode decode each; in
+// FP64 the rows go in fours (v_mfma_f64_4x4x4f64), 3 x 48 matrix cycles per variable and step instead of
+// 3 x 80 at p = 3, 3 x 16 instead of 3 x 64 at p = 2.  HLLC residual at 48^3: p = 3 FP32 468 -> 432 us,
+// FP64 777 -> 763 us, p = 2 279 -> 259 us; JVP p = 2 535 -> 510 us, p = 3 FP32 703 -> 689 us.
+template <class TS, typename Real, int V>
+struct QAcc {
+  typedef typename MM<Real>::acc acc_t;
+  static constexpr bool FOUR = std::is_same<Real, double>::value;
+  static constexpr int G = FOUR ? (TS::NP + 3) / 4 : (TS::NP + 15) / 16;
+  typename std::conditional<FOUR, Real, acc_t>::type q[TS::D][V][G];
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int e = 0; e < TS::D; e++)
+#pragma unroll
+      for (int v = 0; v < V; v++)
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+          if constexpr (FOUR) q[e][v][g] = Real(0); else q[e][v][g] = acc_zero<Real>();
+        }
+  }
+  // left operands of a node: nrow its row of the volume table
+  __device__ __forceinline__ static void load(const Real* nrow, int col, Real (&a)[G]) {
+#pragma unroll
+    for (int g = 0; g < G; g++) a[g] = FOUR ? nrow[4 * g + (col & 3)] : nrow[16 * g + col < TS::N ? 16 * g + col : TS::FZERO];
+  }
+  __device__ __forceinline__ void test(const Real (&a)[G], int e, const Real (&g_)[V]) {
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        if constexpr (FOUR) q[e][v][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[g], g_[v], q[e][v][g], 0, 0, 0);
+        else q[e][v][g] = MM<Real>::mma(a[g], g_[v], q[e][v][g]);
+      }
+  }
+};
+
+// racc[v][m] += sum_e D_e[m][n] Q_e,n through `stage` (16 D NP Real of this wavefront's own).
+template <class TS, typename Real, int V>
+__device__ __forceinline__ void q_fold(const Real* tab, Real* stage, int col, int grp, const QAcc<TS, Real, V>& q, TAcc<TS, Real, V>& racc) {
+  typedef QAcc<TS, Real, V> Q;
+#pragma unroll
+  for (int v = 0; v < V; v++) {
+#pragma unroll
+    for (int e = 0; e < TS::D; e++)
+#pragma unroll
+      for (int g = 0; g < Q::G; g++) {
+        if constexpr (Q::FOUR) {
+          const int n = 4 * g + grp;
+          if (n < TS::NP) stage[(e * TS::NP + n) * 16 + col] = q.q[e][v][g];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const int n = 16 * g + MM<Real>::row(grp, r);
+            if (n < TS::NP) stage[(e * TS::NP + n) * 16 + col] = q.q[e][v][g][r];
+          }
+        }
+      }
+    __builtin_amdgcn_wave_barrier();
+    racc.add(v, grp, [&](int m) {
+      const Real* d = tab + TS::O_DT + m * TS::DT;
+      constexpr int NT = TS::P == 3 ? TS::D + 1 : TS::D;
+      Real s = Real(0), x[NT];
+#pragma unroll
+      for (int e = 0; e < NT; e++) { x[e] = stage[(int)d[e] * 16 + col]; s += d[2 * (TS::D + 1) + e] * x[e]; }
+#pragma unroll
+      for (int e = 0; e < NT; e++) s += d[TS::D + 1 + e] * x[e];
+      return s;
+    });
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <class TS, typename Real>
 __device__ __forceinline__ Real vol_weight(const Real* tab, const int (&q)[3]) {
   const Real* w = tab + TS::O_W;
   if (TS::D == 3) return (w[q[2]] * w[q[1]]) * w[q[0]];
@@ -318,6 +421,13 @@ template <int D, bool H> struct HandAdjoint<FormEuler<D, H>> : std::true_type {}
 template <class Form> struct IsHLLC : std::false_type {};
 template <int D> struct IsHLLC<FormEuler<D, true>> : std::true_type {};
 
+// Residual and JVP kernels of the Euler forms that use the volume table and the projected volume test
+// (QAcc).  Not the cell-split forms, whose workgroups would load the table for a quarter of the work
+// (p = 3 JVP, 12^3: 55 us without, 61 us with), nor the VJP kernels, whose registers are full (p = 3 fused,
+// 48^3: FP64 1640 / 1650 us, FP32 993 / 1642 us).
+template <class Form, bool SPLIT>
+constexpr bool euler_projects() { return HandAdjoint<Form>::value && !SPLIT; }
+
 constexpr int TWAVES = 4;
 
 // Cell-split form of the Euler kernels (SPLIT): the TWAVES wavefronts of a workgroup share one group
@@ -383,6 +493,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   constexpr bool TAN = (MODE == MODE_JVP);
   constexpr int NARR = TAN ? 2 : 1;
   constexpr int STRIDE = NT | 1;
+  constexpr bool PROJ = euler_projects<Form, SPLIT>();   // volume table and projected volume test
   typedef typename std::conditional<TAN, Dual<1, Real>, Real>::type T;
 
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -396,6 +507,8 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   // face tables: traces, and the reference-derivative traces where the faces use gradients
   Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * NARR * 16 * STRIDE;
   ft_load<TS>(ft, a.tab, form_face_tables<Form, D>());
+  Real* vt = ft + form_face_tables<Form, D>() * TS::FTAB;
+  if (PROJ) vt_load<TS>(vt, a.tab);
   stage16<Real, NT>(stU, STRIDE, a.U, cell0, a.J, lane);
   if (TAN) stage16<Real, NT>(stX, STRIDE, a.X, cell0, a.J, lane);
   __syncthreads();
@@ -421,12 +534,15 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   auto Bx = [&](int v, int kk) { int m = 4 * kk + grp; return ownX[v * N + (m < N ? m : N - 1)] * ((m < N) ? sc : Real(0)); };
 
   // ------------------------------------------------------------------ volume
+  QAcc<TS, Real, PROJ ? V : 1> qacc;
+  qacc.zero();
   for (int t = SPLIT ? wave : 0; t < TS::TV; t += SPLIT ? TWAVES : 1) {
     int qe[3];
     const int nodeE = t * 16 + col;
     vol_axes<D, K1>(nodeE < TS::KV ? nodeE : 0, qe);
     acc_t u[V], du[V], gu[D][V], dgu[D][V];
-    t_eval<TS, Real, V>(tab, qe, -1, grp, Bu, u);
+    if constexpr (PROJ) t_eval_ft<TS, Real, V>(vt + nodeE * TS::FS + grp, Bu, u);
+    else t_eval<TS, Real, V>(tab, qe, -1, grp, Bu, u);
     if (TAN) t_eval<TS, Real, V>(tab, qe, -1, grp, Bx, du);
     if (Form::VOL_GRADU) {
 #pragma unroll
@@ -460,6 +576,8 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
         }
       }
       Form::template volume<D, T, Real>(a.fp, Uq, GU, F);
+      Real qa[QAcc<TS, Real, PROJ ? V : 1>::G];
+      if (PROJ) QAcc<TS, Real, PROJ ? V : 1>::load(vt + node * TS::FS, col, qa);
 #pragma unroll
       for (int e = 0; e < D; e++) {
         Real g[V];
@@ -472,10 +590,13 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
           }
           g[v] = pad ? Real(0) : s * wq;
         }
-        t_test<TS, Real, V>(tab, q, e, col, g, racc);
+        if constexpr (PROJ) qacc.test(qa, e, g);
+        else t_test<TS, Real, V>(tab, q, e, col, g, racc);
       }
     }
   }
+
+  if constexpr (PROJ) q_fold<TS, Real, V>(tab, vt + TS::VTAB + wave * (16 * D * TS::NP), col, grp, qacc, racc);
 
   // ------------------------------------------------------------------- faces
   const Real pbd = Real(a.fp.penalty_base * a.fp.penalty_deg);
@@ -952,8 +1073,9 @@ constexpr size_t kt_lds_bytes(int narrays) {
 // kt_forward and kt_adjoint: the same, followed by their face tables
 template <class Form, int D, int P, int K1, typename Real>
 constexpr size_t kt_forward_lds_bytes(int narrays) {
-  return kt_lds_bytes<D, P, K1, Form::V, Real>(narrays) +
-         (size_t)form_face_tables<Form, D>() * TShape<D, P, K1>::FTAB * sizeof(Real);
+  typedef TShape<D, P, K1> TS;
+  const size_t proj = HandAdjoint<Form>::value ? TS::VTAB + TWAVES * 16 * D * TS::NP : 0;   // volume table, q_fold staging
+  return kt_lds_bytes<D, P, K1, Form::V, Real>(narrays) + (form_face_tables<Form, D>() * TS::FTAB + proj) * sizeof(Real);
 }
 
 }  // namespace bosss
@@ -1258,7 +1380,10 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   Real* tab = reinterpret_cast<Real*>(smem_raw);
   Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * NSLOT * 64;
   for (int i = threadIdx.x; i < TS::TAB; i += blockDim.x) tab[i] = a.tab[i];
-  ft_load<TS>(ft, a.tab);
+  // FP64 p = 3 has no registers left for it (48^3: 1260 us without, 1368 us with, spilling)
+  constexpr bool PROJ = euler_projects<Form, SPLIT>() && (sizeof(Real) == 4 || P < 3);
+  if (PROJ) vt_load<TS>(ft, a.tab);   // the volume table first; the face table takes its place
+  else ft_load<TS>(ft, a.tab);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -1324,14 +1449,22 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   };
 
   // ------------------------------------------------------------------ volume
+  const Real* vt = ft;
+  QAcc<TS, Real, PROJ ? V : 1> qacc;
+  qacc.zero();
   for (int t = SPLIT ? wave : 0; t < TS::TV; t += SPLIT ? TWAVES : 1) {
     int qe[3];
     const int nodeE = t * 16 + col;
     vol_axes<D, K1>(nodeE < TS::KV ? nodeE : 0, qe);
     // state and tangent at the nodes are used once each: read straight from the MFMA results
     acc_t au[V], adu[V];
-    t_eval<TS, Real, V>(tab, qe, -1, grp, Bu, au);
-    t_eval<TS, Real, V>(tab, qe, -1, grp, Bx, adu);
+    if constexpr (PROJ) {
+      t_eval_ft<TS, Real, V>(vt + nodeE * TS::FS + grp, Bu, au);
+      t_eval_ft<TS, Real, V>(vt + nodeE * TS::FS + grp, Bx, adu);
+    } else {
+      t_eval<TS, Real, V>(tab, qe, -1, grp, Bu, au);
+      t_eval<TS, Real, V>(tab, qe, -1, grp, Bx, adu);
+    }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       if (t * 16 + MM<Real>::row(0, r) >= TS::KV) continue;   // all 4 nodes of this step are padding
@@ -1349,6 +1482,8 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
         for (int d = 0; d < D; d++) GU[v][d] = Uq[v];
       }
       Form::template volume<D, T, Real>(a.fp, Uq, GU, F);
+      Real qa[QAcc<TS, Real, PROJ ? V : 1>::G];
+      if (PROJ) QAcc<TS, Real, PROJ ? V : 1>::load(vt + node * TS::FS, col, qa);
 #pragma unroll
       for (int e = 0; e < D; e++) {
         Real g[V];
@@ -1359,9 +1494,17 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
           for (int d = 0; d < D; d++) s += F[v][d].d[0] * iJ[e][d];
           g[v] = pad ? Real(0) : s * wq;
         }
-        t_test<TS, Real, V>(tab, q, e, col, g, racc);
+        if constexpr (PROJ) qacc.test(qa, e, g);
+        else t_test<TS, Real, V>(tab, q, e, col, g, racc);
       }
     }
+  }
+
+  if constexpr (PROJ) {
+    q_fold<TS, Real, V>(tab, buf, col, grp, qacc, racc);
+    __syncthreads();
+    ft_load<TS>(ft, a.tab);
+    __syncthreads();
   }
 
   // ------------------------------------------------------------------- faces
