@@ -70,6 +70,7 @@ SIGNATURES = {
     "bosss_hip_evaluate_dev": (ctypes.c_int, [_vp, ctypes.c_double, ctypes.c_double, _vp, _vp, _vp]),
     "bosss_hip_jvp_dev": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp]),
     "bosss_hip_vjp_dev": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp]),
+    "bosss_hip_combine_dev": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_vp), _vp, _vp, _vp]),
     "bosss_hip_evaluate_vjp_dev": (ctypes.c_int, [_vp, ctypes.c_double, ctypes.c_double, _vp, _vp, _vp, _vp, _vp]),
     "bosss_hip_op_matrix_layout": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64),
                                                   ctypes.POINTER(ctypes.c_int32), _vp]),

@@ -195,6 +195,14 @@ class DifferentialOperator:
         check(lib().bosss_hip_evaluate_vjp_dev(self.h, alpha, beta, self._ptr(U), self._ptr(R), self._ptr(W), self._ptr(out),
                                                self._stream(stream)))
 
+    def combine_dev(self, y, coefs, ks, out, stream=None):
+        """out <- y + sum_i coefs[i] ks[i] in one pass (out may be y, but none of ks)."""
+        self._check_dev(y, out, *ks)
+        n = len(ks)
+        if len(coefs) != n or any(k.data_ptr() == out.data_ptr() for k in ks):
+            raise ValueError("one coefficient per vector, and out none of them")
+        check(lib().bosss_hip_combine_dev(self.h, n, (ctypes.c_double * n)(*coefs), (ctypes.c_void_p * n)(*[k.data_ptr() for k in ks]),
+                                          self._ptr(y), self._ptr(out), self._stream(stream)))
 
     # ------------------------------------------------ operator matrix (block-ELL)
     def matrix_layout(self):
@@ -212,8 +220,7 @@ class DifferentialOperator:
 
     def diag_blocks_dev(self, U, blocks, alpha=1.0, shift=0.0, transposed=False, stream=None):
         """blocks <- alpha * dR_j/dU_j(U) + shift * I for every cell j: J row-major Nt x Nt FP64
-        blocks, or each block transposed (own-cell JVP probes in the operator's precision; U is a
-        state vector of it)."""
+        blocks, or each block transposed (U is a state vector in the operator's precision)."""
         import torch
         self._check_dev(U)
         Nt = self.nvars * self.N

@@ -34,7 +34,7 @@ class RungeKutta:
         self.U = U                                   # current state, updated in place
         self.time = 0.0
         self.k = [torch.empty_like(U) for _ in range(scheme.stages)]
-        self.y0 = torch.empty_like(U)
+        self.y = torch.empty_like(U)                 # stage states
 
     def ComputeChangeRate(self, k, U):
         """k += R(U)  (ExplicitEuler.ComputeChangeRate)."""
@@ -43,19 +43,24 @@ class RungeKutta:
     def Perform(self, dt):
         """One time step of size dt; returns dt (RungeKutta.Perform)."""
         sch = self.scheme
-        self.y0.copy_(self.U)
+        overridden = type(self).ComputeChangeRate is not RungeKutta.ComputeChangeRate
         for s in range(sch.stages):
-            if s > 0:
-                # PerformStage: U = y0 - dt sum_r a[s][r] k[r]
-                self.U.copy_(self.y0)
-                for r in range(s):
-                    if sch.a[s][r] != 0.0:
-                        self.U.add_(self.k[r], alpha=-dt * sch.a[s][r])
-            self.k[s].zero_()
-            self.ComputeChangeRate(self.k[s], self.U)
-        self.U.copy_(self.y0)
-        for s in range(sch.stages):
-            if sch.b[s] != 0.0:
-                self.U.add_(self.k[s], alpha=-dt * sch.b[s])
+            # PerformStage: y = U - dt sum_r a[s][r] k[r]
+            y = self._combine(sch.a[s][:s], dt, self.y)
+            if overridden:
+                self.k[s].zero_()
+                self.ComputeChangeRate(self.k[s], y)
+            else:
+                self.op.evaluate_dev(y, self.k[s])   # its first write: no zeros to add to
+        self._combine(sch.b, dt, self.U)
         self.time += dt
         return dt
+
+    def _combine(self, a, dt, out):
+        """out <- U - dt sum_r a[r] k[r] over the coefficients that are not zero; returns where the result is
+        (U itself if there are none)."""
+        used = [r for r in range(len(a)) if a[r] != 0.0]
+        if not used:
+            return self.U
+        self.op.combine_dev(self.U, [-dt * a[r] for r in used], [self.k[r] for r in used], out)
+        return out
