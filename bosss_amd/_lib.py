@@ -70,7 +70,6 @@ SIGNATURES = {
     "bosss_hip_evaluate_dev": (ctypes.c_int, [_vp, ctypes.c_double, ctypes.c_double, _vp, _vp, _vp]),
     "bosss_hip_jvp_dev": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp]),
     "bosss_hip_vjp_dev": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp]),
-    "bosss_hip_combine_dev": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_vp), _vp, _vp, _vp]),
     "bosss_hip_evaluate_vjp_dev": (ctypes.c_int, [_vp, ctypes.c_double, ctypes.c_double, _vp, _vp, _vp, _vp, _vp]),
     "bosss_hip_op_matrix_layout": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64),
                                                   ctypes.POINTER(ctypes.c_int32), _vp]),
@@ -124,6 +123,11 @@ SIGNATURES = {
                                            ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32), _dp]),
 }
 
+# Calls of this package's own steppers, not part of the C interface (include/bosss_hip.h).
+INTERNAL = {
+    "bosss_internal_combine": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_vp), _vp, _vp, _vp]),
+}
+
 _lib = None
 
 
@@ -148,7 +152,7 @@ def lib():
         except ImportError:
             pass
         L = ctypes.CDLL(LIBPATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **INTERNAL}.items():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

@@ -775,7 +775,10 @@ static void launch_combine(int nk, int64_t nv, const CombineArgs& a, const void*
 
 extern "C" {
 
-int bosss_hip_combine_dev(bosss_op* op, int32_t nk, const double* coef, const double* const* k, const double* y, double* out,
+// out <- y + sum_i coef[i] k[i], in index order, for vectors of the operator (ndof entries of its
+// precision): the updates of an explicit Runge-Kutta step (RungeKutta.cs:242-310).  coef and k are host
+// arrays of nk entries; out may be y, no k[i] may be out.
+int bosss_internal_combine(bosss_op* op, int32_t nk, const double* coef, const double* const* k, const double* y, double* out,
                           void* stream) {
   if (!op || !y || !out || nk < 0 || (nk && (!coef || !k))) return fail(BOSSS_ERR_ARG, "NULL argument");
   for (int i = 0; i < nk; i++)

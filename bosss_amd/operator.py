@@ -201,7 +201,7 @@ class DifferentialOperator:
         n = len(ks)
         if len(coefs) != n or any(k.data_ptr() == out.data_ptr() for k in ks):
             raise ValueError("one coefficient per vector, and out none of them")
-        check(lib().bosss_hip_combine_dev(self.h, n, (ctypes.c_double * n)(*coefs), (ctypes.c_void_p * n)(*[k.data_ptr() for k in ks]),
+        check(lib().bosss_internal_combine(self.h, n, (ctypes.c_double * n)(*coefs), (ctypes.c_void_p * n)(*[k.data_ptr() for k in ks]),
                                           self._ptr(y), self._ptr(out), self._stream(stream)))
 
     # ------------------------------------------------ operator matrix (block-ELL)

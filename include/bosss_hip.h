@@ -144,11 +144,6 @@ int bosss_hip_vjp_dev(bosss_op* op, const double* U, const double* W, double* Jt
 /* fused: R <- beta*R + alpha*Op(U) and JtW <- J(U)^T W in one pass over U */
 int bosss_hip_evaluate_vjp_dev(bosss_op* op, double alpha, double beta, const double* U, double* R, const double* W,
                                double* JtW, void* stream);
-/* out <- y + sum_i coef[i] k[i], in index order, for vectors of the operator (ndof entries of its
- * precision): the stage and final updates of an explicit Runge-Kutta step in one pass (RungeKutta.cs:242-310).
- * coef and k are host arrays of nk entries; out may be y, no k[i] may be out. */
-int bosss_hip_combine_dev(bosss_op* op, int32_t nk, const double* coef, const double* const* k, const double* y, double* out,
-                          void* stream);
 
 /* ---- operator matrix (replaces EvaluatorLinear.ComputeMatrix, DifferentialOperator.cs:1721-1838,
  *      into a BlockMsrMatrix, BlockMsrMatrix.cs:186/1388, and the coloured

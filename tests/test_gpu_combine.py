@@ -1,4 +1,4 @@
-"""bosss_hip_combine_dev: out = y + sum c_i k_i, one to nine vectors, odd lengths and unaligned vectors."""
+"""DifferentialOperator.combine_dev: out = y + sum c_i k_i, one to nine vectors, odd lengths and unaligned vectors."""
 import pytest
 
 pytestmark = pytest.mark.gpu
