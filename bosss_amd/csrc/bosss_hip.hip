@@ -132,13 +132,45 @@ __global__ void __launch_bounds__(256) k_axis_arrays(int J, int D, const double*
     anb[(size_t)f * J + j] = nb[(size_t)j * NF + f];
   }
 }
+// Clears *axis unless every cell is axis-aligned: invJ diagonal and positive, the normal of face f the
+// unit vector of its axis and side.
+__global__ void __launch_bounds__(256) k_axis_check(int J, int D, const double* __restrict__ invJ, const double* __restrict__ normal,
+                                                    int* __restrict__ axis) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x, NF = 2 * D;
+  if (j >= J) return;
+  bool ok = true;
+  for (int e = 0; e < D; e++)
+    for (int d = 0; d < D; d++) {
+      const double v = invJ[((size_t)j * D + e) * D + d];
+      ok = ok && (e == d ? v > 0.0 : v == 0.0);
+    }
+  for (int f = 0; f < NF; f++)
+    for (int d = 0; d < D; d++)
+      ok = ok && normal[((size_t)j * NF + f) * D + d] == (d == face_dir(f) ? (face_upper(f) ? 1.0 : -1.0) : 0.0);
+  if (!ok) *axis = 0;   // any number of threads, the same value
+}
 static int make_axis_arrays(bosss_grid* G) {
+  for (int f = 0; f < G->NF; f++)   // opposite faces paired
+    if (face_dir(G->pair[f]) != face_dir(f) || face_upper(G->pair[f]) == face_upper(f)) return BOSSS_OK;
   const size_t J = G->J;
-  HIPCHK(hipMalloc((void**)&G->axis_real, (size_t)(G->D + G->NF) * J * sizeof(double)));
-  HIPCHK(hipMalloc((void**)&G->axis_nb, (size_t)G->NF * J * sizeof(int)));
+  const dim3 grid((unsigned)((J + 255) / 256));
   hipStream_t s = G->ctx->stream;
-  hipLaunchKernelGGL(k_axis_arrays, dim3((unsigned)((J + 255) / 256)), dim3(256), 0, s, G->J, G->D, G->invJ, G->sqrtg, G->nb,
-                     G->axis_real, G->axis_nb);
+  int axis = 1, rc;
+  HIPCHK(hipMalloc((void**)&G->axis_real, (size_t)(G->D + G->NF) * J * sizeof(double)));
+  if ((rc = upload(&G->axis_nb, (const int*)nullptr, (size_t)G->NF * J))) return rc;
+  HIPCHK(hipMemcpyAsync(G->axis_nb, &axis, sizeof axis, hipMemcpyHostToDevice, s));   // the flag, until the arrays are made
+  hipLaunchKernelGGL(k_axis_check, grid, dim3(256), 0, s, G->J, G->D, G->invJ, G->normal, G->axis_nb);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(&axis, G->axis_nb, sizeof axis, hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  if (!axis) {
+    HIPCHK(hipFree(G->axis_real));
+    G->axis_real = nullptr;
+    HIPCHK(hipFree(G->axis_nb));
+    G->axis_nb = nullptr;
+    return BOSSS_OK;
+  }
+  hipLaunchKernelGGL(k_axis_arrays, grid, dim3(256), 0, s, G->J, G->D, G->invJ, G->sqrtg, G->nb, G->axis_real, G->axis_nb);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));   // any stream may read them after the upload returns
   return BOSSS_OK;
@@ -254,21 +286,6 @@ int bosss_hip_grid_upload(bosss_ctx* ctx, const bosss_grid_desc* g, bosss_grid**
   for (const auto& oc : offsets)
     if (2LL * oc.second >= J) plane = std::max(plane, oc.first);
 
-  // Axis-aligned: invJ diagonal and positive, the normal of face f the unit vector of its axis and
-  // side, and opposite faces paired, on every cell.
-  bool axis = true;
-  for (int f = 0; f < NF && axis; f++) axis = face_dir(pair[f]) == face_dir(f) && face_upper(pair[f]) != face_upper(f);
-  for (int j = 0; j < J && axis; j++) {
-    for (int e = 0; e < D; e++)
-      for (int d = 0; d < D; d++) {
-        const double v = g->invJ[((size_t)j * D + e) * D + d];
-        axis = axis && (e == d ? v > 0.0 : v == 0.0);
-      }
-    for (int f = 0; f < NF; f++)
-      for (int d = 0; d < D; d++)
-        axis = axis && nrm[((size_t)j * NF + f) * D + d] == (d == face_dir(f) ? (face_upper(f) ? 1.0 : -1.0) : 0.0);
-  }
-
   HIPCHK(hipSetDevice(ctx->device));
   bosss_grid* G = new bosss_grid();
   G->ctx = ctx; G->D = D; G->J = J; G->E = E; G->NF = NF; G->has_boundary = has_boundary;
@@ -279,7 +296,7 @@ int bosss_hip_grid_upload(bosss_ctx* ctx, const bosss_grid_desc* g, bosss_grid**
   if ((rc = upload(&G->detJ, g->detJ, J)) || (rc = upload(&G->invJ, g->invJ, (size_t)J * D * D)) ||
       (rc = upload(&G->scaling, g->scaling, J)) || (rc = upload(&G->lenscale, g->lenscale, J)) ||
       (rc = upload(&G->nb, nb.data(), nb.size())) || (rc = upload(&G->sqrtg, sg.data(), sg.size())) ||
-      (rc = upload(&G->normal, nrm.data(), nrm.size())) || (axis && (rc = make_axis_arrays(G)))) {
+      (rc = upload(&G->normal, nrm.data(), nrm.size())) || (rc = make_axis_arrays(G))) {
     bosss_hip_grid_destroy(G);
     return rc;
   }
@@ -983,11 +1000,15 @@ static int assemble_linear(bosss_op* op, int S, double alpha, double beta, doubl
 static int euler_blocks(bosss_op* op, const void* U, double alpha, double shift, int transposed, double* blocks, hipStream_t s) {
   const bosss_grid* g = op->grid;
   const int P = op->ks->P;
+  // 3D alone: the 24 columns of the 2D p = 2 blocks cost little by probing, and by moments they measured
+  // 12 % further from 64-bit exact (7.1e-16 against 6.3e-16; 3D p = 2 8.5e-16 against 9.0e-16, p = 3
+  // 1.4e-15 against 1.7e-15)
+  if (op->D != 3) return BOSSS_ERR_UNSUPPORTED;
   if (!op->d_ebreal) {
     std::vector<double> x, w;
     gauss_legendre(op->K1, x, w);
     EulerBlockTables t;
-    euler_block_tables(op->D, P, op->K1, x, w, t);
+    euler_block_tables(op->D, P, op->K1, x, t);
     int rc;
     if ((!op->d_ebints && (rc = upload(&op->d_ebints, t.ints.data(), t.ints.size()))) ||
         (rc = upload(&op->d_ebreal, t.real.data(), t.real.size())))
@@ -1121,8 +1142,8 @@ int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, doub
   HIPCHK(hipSetDevice(op->ctx->device));
   hipStream_t s = (hipStream_t)stream;
   if (!op->lin_host.empty()) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
-  // Euler forms on tensor tables: directly, unless no kernel is built for them; operators on general
-  // tables go through the probes (20^3, p = 3: 17.4 ms by 100 probes, 1.18 ms directly).
+  // Euler forms on tensor tables: directly, unless no kernel is built for them (2D); those and operators
+  // on general tables go through the probes (20^3, p = 3: 17.4 ms by 100 probes, 1.18 ms directly).
   if (op->tensor && (rc = euler_blocks(op, U, alpha, shift, (int)(transposed != 0), blocks, s)) != BOSSS_ERR_UNSUPPORTED) return rc;
   if ((rc = ensure_staging(op))) return rc;
   const int J = op->grid->J, Nt = op->V * op->N;

@@ -14,7 +14,7 @@ struct EulerBlockTables {
   std::vector<double> real;    // 1D values, volume and face moment matrices in MFMA order, term coefficients
   std::vector<int32_t> ints;   // term list offsets, entry order, term indices
 };
-void euler_block_tables(int D, int P, int K1, const std::vector<double>& x, const std::vector<double>& w, EulerBlockTables& t);
+void euler_block_tables(int D, int P, int K1, const std::vector<double>& nodes, EulerBlockTables& t);   // nodes: 1D Gauss nodes
 
 struct EulerBlockArgs {
   int J;
