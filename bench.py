@@ -412,10 +412,10 @@ def newton_comparison(grid, op64, Un, form, p):
 def implicit_cfl_comparison(grid, op64, Un, form, p, mult=10.0):
     """The same implicit step at mult times the time step (a CFL number mult times larger), where the
     Krylov iterations grow: plain FP64 Newton-GMRES against the cell-block preconditioned variants
-    (blocks of I/dt + dR_j/dU_j from own-cell JVP probes, inverted in FP64): FP64 with the FP64
+    (blocks of I/dt + dR_j/dU_j, inverted in FP64): FP64 with the FP64
     preconditioner, and the FP64 defect correction around FP32 GMRES with the FP32 preconditioner
-    (FP32 probes and apply).  One solve each after a warm-up; the preconditioner set-up (probes,
-    batched LU with inverse, transposition) is timed separately."""
+    (FP32 apply).  One solve each after a warm-up; the preconditioner set-up (blocks and their
+    batched inverse) is timed separately."""
     import torch
     from bosss_amd.blocks import CellBlockPreconditioner
     from bosss_amd.newton import ImplicitStep

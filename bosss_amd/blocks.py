@@ -87,8 +87,7 @@ class CellBlockPreconditioner:
     block-Jacobi of a Newton-Krylov step (BlockJacobi.InitImpl / Solve, BlockJacobi.cs:63-197, on the
     diagonal blocks of the linearised operator), without assembling the off-diagonal blocks.
 
-    The blocks come from own-cell JVP probes of ``op`` (``bosss_hip_op_diag_blocks_dev``; an FP32
-    operator probes in FP32) in transposed storage, which the probes write contiguously; inverting
+    The blocks come from ``bosss_hip_op_diag_blocks_dev`` in transposed storage; inverting
     D^T in place in FP64 (batched LU pivots, Gauss-Jordan inverse) gives (D^-1)^T, the layout in
     which the apply (``bosss_hip_block_gemv_uniform_dev``) reads each block column by column,
     coalesced; it is kept in the apply precision ("fp32": rounded once to FP32)."""
