@@ -19,7 +19,7 @@
 //
 // Bound: HBM and L2 traffic (own and 2D neighbour coefficients, one store), where the nodal kernels
 // of dg_tensor.hpp are bound by their dense contractions.  Upwind + SIP p = 3 residual at 64^3, FP64:
-// 522 us by the nodal kernel, 44 us here (84 MB of coefficients in and out, 31 MB of metrics); FP32
+// 522 us by the nodal kernel, 47 us here (84 MB of coefficients in and out, 31 MB of metrics); FP32
 // adjoint at 45 x 37 x 29: 65 -> 9.5 us, the cost of the call.  Measured and not kept: all faces
 // unrolled (448 registers, 60 us), neighbour coefficients gathered through an LDS tile (67 us: the
 // lane exchange of the cell indices costs more than the scattered lines), results stored without
