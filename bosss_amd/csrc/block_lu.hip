@@ -1185,23 +1185,51 @@ __global__ void __launch_bounds__(64) k_lu_first_zero(int nblk, int nmax, const 
   if (threadIdx.x == 0) info[b] = inf;
 }
 
-// x_b <- LU_b \ x_b   (getrs with the 1-based pivots), two kernels that each take their block sizes.
+// x_b <- LU_b \ x_b   (getrs with the 1-based pivots), two kernels that each take their block sizes; any size.
 //
 // Up to SOLVE_SMALL DOF: one wavefront per block, lane l holds x_l and x_64+l in registers.  The
 // substitutions run column by column; the finished x_j reaches the other lanes as a scalar and the
 // factor's columns, which do not depend on it, are loaded ahead.  The forward sweep adds the terms of a
 // row in getrs' order (k = 0 .. i-1), the backward sweep from the last column.
 //
-// Above: one workgroup per block, x in LDS, SOLVE_T columns at a time: one wavefront solves the diagonal
+// Up to LU_BIG_MAXN, the largest x that LDS holds: one workgroup per block, x in LDS, SOLVE_T columns at a time: one wavefront solves the diagonal
 // tile, staged in LDS, then every wavefront subtracts the finished entries from groups of 64 rows, lane
 // by lane in the same order.  The factor does not depend on x, so the next tile and every wavefront's
 // first group are loaded (coalesced, turned in LDS) while the diagonal tile is solved.
+//
+// Above (factors that were made elsewhere): one wavefront per block, x in place (solve_in_memory).
 //
 // Bound: the 2 n dependent steps of the diagonal tiles, half of them with a division.  48 blocks of
 // 200..540 DOF: 1.67 ms by one wavefront per block walking the factor's columns in memory, 0.20 ms here;
 // 300 of 100 DOF 0.14 -> 0.08 ms.  Measured and not kept: lane partial sums of the rows (0.20 ms too, and
 // other rounding), the division by a Newton step on a reciprocal (0.23 ms).
 constexpr int SOLVE_SMALL = 128, SOLVE_T = 64, SOLVE_WAVES = 8;
+
+// One wavefront, lane l owns the rows l (mod 64) of x and is the only one to write them; column by column,
+// the finished x_j reaches the other lanes by a shuffle from its owner.
+__device__ void solve_in_memory(int n, const double* __restrict__ L, const int32_t* __restrict__ pv, double* x) {
+  const int lane = threadIdx.x;
+  if (lane == 0)
+    for (int j = 0; j < n; j++) {
+      const int p = pv[j] - 1;
+      if (p != j) { const double t = x[j]; x[j] = x[p]; x[p] = t; }
+    }
+  __syncthreads();   // the interchanged entries are read by their owners below
+  for (int j = 0; j < n; j++) {
+    double xj = lane == (j & 63) ? x[j] : 0.0;
+    xj = __shfl(xj, j & 63, 64);
+    for (int i = lane + (lane <= j ? ((j - lane) / 64 + 1) * 64 : 0); i < n; i += 64) x[i] -= L[(size_t)i * n + j] * xj;
+  }
+  for (int j = n - 1; j >= 0; j--) {
+    double xj = 0.0;
+    if (lane == (j & 63)) {
+      xj = x[j] / L[(size_t)j * n + j];
+      x[j] = xj;
+    }
+    xj = __shfl(xj, j & 63, 64);
+    for (int i = lane; i < j; i += 64) x[i] -= L[(size_t)i * n + j] * xj;
+  }
+}
 
 __global__ void __launch_bounds__(64) k_block_solve(int nblk, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
                                                     const double* __restrict__ LU, const int32_t* __restrict__ ipiv,
@@ -1210,7 +1238,11 @@ __global__ void __launch_bounds__(64) k_block_solve(int nblk, const int32_t* __r
   const int b = blockIdx.x;
   if (b >= nblk) return;
   const int n = nsz[b];
-  if (n <= 0 || n > SOLVE_SMALL) return;
+  if (n <= 0 || (n > SOLVE_SMALL && n <= LU_BIG_MAXN)) return;
+  if (n > LU_BIG_MAXN) {
+    solve_in_memory(n, LU + off[b], ipiv + pivoff[b], x + xoff[b]);
+    return;
+  }
   const int lane = threadIdx.x;
   const double* L = LU + off[b];
   const int32_t* pv = ipiv + pivoff[b];
