@@ -9,6 +9,7 @@
 #include <cstring>
 #include <initializer_list>
 #include <map>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -70,9 +71,11 @@ struct bosss_grid {
   double* normal;   // [J][NF][D]
   int pair[6];
   // axis-aligned cells (diagonal invJ, unit normals along the faces' axes): the same metrics in
-  // cell-fastest arrays, in one allocation each; nullptr otherwise
-  double* axis_real;   // [D][J] invJ diagonal, [NF][J] sqrtg
-  int* axis_nb;        // [NF][J]
+  // cell-fastest arrays, made for the first operator that reads them (axis_arrays); nullptr otherwise
+  mutable std::mutex axis_lock;
+  mutable bool axis_known = false;
+  mutable double* axis_real = nullptr;   // [D][J] invJ diagonal, [NF][J] sqrtg
+  mutable int* axis_nb = nullptr;        // [NF][J]
 };
 
 struct bosss_op {
@@ -84,6 +87,8 @@ struct bosss_op {
   void* ttab;        // 1D tensor tables (Real) on the device, if the uploaded tables are a tensor product
   bool tensor;
   bool split[KernelSet::NVARIANT] = {false, false, false, false};   // cell-split kernels (split_pays)
+  const double* axis_real = nullptr;   // the grid's cell-fastest metrics, if the modal kernels run
+  const int* axis_nb = nullptr;
   FormParams fp;
   size_t ndof;
   // staging buffers for the host-pointer entry points
@@ -120,22 +125,11 @@ int bell_default_nl(int Nt);
 void bell_candidates(int Nt, std::vector<int>& out);
 }
 
-// The cell-fastest copies of the metrics of an axis-aligned grid, made on the device from the
-// uploaded arrays.
+// The cell-fastest copies of a grid's metrics, and *skew = 1 unless every cell is axis-aligned: invJ
+// diagonal and positive, the normal of face f the unit vector of its axis and side.
 __global__ void __launch_bounds__(256) k_axis_arrays(int J, int D, const double* __restrict__ invJ, const double* __restrict__ sqrtg,
-                                                     const int* __restrict__ nb, double* __restrict__ real, int* __restrict__ anb) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x, NF = 2 * D;
-  if (j >= J) return;
-  for (int d = 0; d < D; d++) real[(size_t)d * J + j] = invJ[((size_t)j * D + d) * D + d];
-  for (int f = 0; f < NF; f++) {
-    real[(size_t)(D + f) * J + j] = sqrtg[(size_t)j * NF + f];
-    anb[(size_t)f * J + j] = nb[(size_t)j * NF + f];
-  }
-}
-// Clears *axis unless every cell is axis-aligned: invJ diagonal and positive, the normal of face f the
-// unit vector of its axis and side.
-__global__ void __launch_bounds__(256) k_axis_check(int J, int D, const double* __restrict__ invJ, const double* __restrict__ normal,
-                                                    int* __restrict__ axis) {
+                                                     const double* __restrict__ normal, const int* __restrict__ nb,
+                                                     double* __restrict__ real, int* __restrict__ anb, int* __restrict__ skew) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x, NF = 2 * D;
   if (j >= J) return;
   bool ok = true;
@@ -143,36 +137,50 @@ __global__ void __launch_bounds__(256) k_axis_check(int J, int D, const double* 
     for (int d = 0; d < D; d++) {
       const double v = invJ[((size_t)j * D + e) * D + d];
       ok = ok && (e == d ? v > 0.0 : v == 0.0);
+      if (e == d) real[(size_t)d * J + j] = v;
     }
-  for (int f = 0; f < NF; f++)
+  for (int f = 0; f < NF; f++) {
     for (int d = 0; d < D; d++)
       ok = ok && normal[((size_t)j * NF + f) * D + d] == (d == face_dir(f) ? (face_upper(f) ? 1.0 : -1.0) : 0.0);
-  if (!ok) *axis = 0;   // any number of threads, the same value
-}
-static int make_axis_arrays(bosss_grid* G) {
-  for (int f = 0; f < G->NF; f++)   // opposite faces paired
-    if (face_dir(G->pair[f]) != face_dir(f) || face_upper(G->pair[f]) == face_upper(f)) return BOSSS_OK;
-  const size_t J = G->J;
-  const dim3 grid((unsigned)((J + 255) / 256));
-  hipStream_t s = G->ctx->stream;
-  int axis = 1, rc;
-  HIPCHK(hipMalloc((void**)&G->axis_real, (size_t)(G->D + G->NF) * J * sizeof(double)));
-  if ((rc = upload(&G->axis_nb, (const int*)nullptr, (size_t)G->NF * J))) return rc;
-  HIPCHK(hipMemcpyAsync(G->axis_nb, &axis, sizeof axis, hipMemcpyHostToDevice, s));   // the flag, until the arrays are made
-  hipLaunchKernelGGL(k_axis_check, grid, dim3(256), 0, s, G->J, G->D, G->invJ, G->normal, G->axis_nb);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(&axis, G->axis_nb, sizeof axis, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  if (!axis) {
-    HIPCHK(hipFree(G->axis_real));
-    G->axis_real = nullptr;
-    HIPCHK(hipFree(G->axis_nb));
-    G->axis_nb = nullptr;
-    return BOSSS_OK;
+    real[(size_t)(D + f) * J + j] = sqrtg[(size_t)j * NF + f];
+    anb[(size_t)f * J + j] = nb[(size_t)j * NF + f];
   }
-  hipLaunchKernelGGL(k_axis_arrays, grid, dim3(256), 0, s, G->J, G->D, G->invJ, G->sqrtg, G->nb, G->axis_real, G->axis_nb);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(s));   // any stream may read them after the upload returns
+  if (!ok) *skew = 1;   // any number of threads, the same value
+}
+// Makes them for an operator of this grid, once; the grid may be shared by threads.  Only the modal kernels
+// read them: 96 bytes per cell in 3D that other operators' grids do not hold.
+static int axis_arrays(const bosss_grid* G) {
+  std::lock_guard<std::mutex> lock(G->axis_lock);
+  if (G->axis_known) return BOSSS_OK;
+  for (int f = 0; f < G->NF; f++)   // opposite faces paired
+    if (face_dir(G->pair[f]) != face_dir(f) || face_upper(G->pair[f]) == face_upper(f)) {
+      G->axis_known = true;
+      return BOSSS_OK;
+    }
+  const size_t J = G->J, nreal = (size_t)(G->D + G->NF) * J, nnb = (size_t)G->NF * J;
+  hipStream_t s = G->ctx->stream;
+  double* real = nullptr;
+  int *anb = nullptr, skew = 0;
+  hipError_t e = hipMalloc((void**)&real, nreal * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc((void**)&anb, (nnb + 1) * sizeof(int));   // the flag behind the neighbours
+  if (e == hipSuccess) e = hipMemsetAsync(anb + nnb, 0, sizeof(int), s);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_axis_arrays, dim3((unsigned)((J + 255) / 256)), dim3(256), 0, s, G->J, G->D, G->invJ, G->sqrtg, G->normal, G->nb,
+                       real, anb, anb + nnb);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(&skew, anb + nnb, sizeof skew, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);   // any stream may read the arrays from here on
+  if (e != hipSuccess || skew) {
+    (void)hipFree(real);
+    (void)hipFree(anb);
+    real = nullptr;
+    anb = nullptr;
+  }
+  HIPCHK(e);
+  G->axis_real = real;
+  G->axis_nb = anb;
+  G->axis_known = true;
   return BOSSS_OK;
 }
 
@@ -296,7 +304,7 @@ int bosss_hip_grid_upload(bosss_ctx* ctx, const bosss_grid_desc* g, bosss_grid**
   if ((rc = upload(&G->detJ, g->detJ, J)) || (rc = upload(&G->invJ, g->invJ, (size_t)J * D * D)) ||
       (rc = upload(&G->scaling, g->scaling, J)) || (rc = upload(&G->lenscale, g->lenscale, J)) ||
       (rc = upload(&G->nb, nb.data(), nb.size())) || (rc = upload(&G->sqrtg, sg.data(), sg.size())) ||
-      (rc = upload(&G->normal, nrm.data(), nrm.size())) || (rc = make_axis_arrays(G))) {
+      (rc = upload(&G->normal, nrm.data(), nrm.size()))) {
     bosss_hip_grid_destroy(G);
     return rc;
   }
@@ -569,6 +577,11 @@ int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tabl
     add(t->face_weights, Ke); add(t->trace, NF * Ke * N); add(t->dtrace, NF * Ke * N * D);
   }
   if ((rc = ks->prepare()) != 0) { bosss_hip_op_destroy(op); return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc); }
+  if (op->tensor && (precision == BOSSS_FP64 ? (const void*)ks->km64[KernelSet::RES] : (const void*)ks->km32[KernelSet::RES])) {
+    if ((rc = axis_arrays(grid)) != BOSSS_OK) { bosss_hip_op_destroy(op); return rc; }
+    op->axis_real = grid->axis_real;
+    op->axis_nb = grid->axis_nb;
+  }
   if (op->tensor)
     for (int i = 0; i < KernelSet::NVARIANT; i++) {
       const void* part = precision == BOSSS_FP64 ? (const void*)ks->kts64[i] : (const void*)ks->kts32[i];
@@ -654,7 +667,7 @@ static int launch_modal(const bosss_op* op, void (*k)(MArgs<Real>), double alpha
   MArgs<Real> a;
   a.J = g->J; a.nxcd = op->ctx->nxcd;
   a.detJ = g->detJ; a.scaling = g->scaling; a.lenscale = g->lenscale;
-  a.g.iJ = g->axis_real; a.g.sqrtg = g->axis_real + (size_t)g->D * g->J; a.g.nb = g->axis_nb;
+  a.g.iJ = op->axis_real; a.g.sqrtg = op->axis_real + (size_t)g->D * g->J; a.g.nb = op->axis_nb;
   a.fp = op->fp; a.alpha = alpha; a.beta = beta;
   a.U = (const Real*)U; a.X = (const Real*)X; a.R = (Real*)R; a.out = (Real*)out;
   hipLaunchKernelGGL(k, dim3((unsigned)((g->J + 63) / 64)), dim3(64), 0, s, a);
@@ -668,9 +681,9 @@ static int launch(bosss_op* op, int which, double alpha, double beta, const void
   HIPCHK(hipSetDevice(op->ctx->device));
   // Linear scalar forms on axis-aligned cells: the modal kernels (own_only probes of these forms
   // do not come here, their diagonal blocks are assembled directly).
-  if (op->tensor && op->grid->axis_nb && op->ks->km64[which] && !own_only) {
+  if (op->axis_nb && !own_only) {
     if (op->precision == BOSSS_FP64) return launch_modal<double>(op, op->ks->km64[which], alpha, beta, U, X, R, out, s);
-    if (op->ks->km32[which]) return launch_modal<float>(op, op->ks->km32[which], alpha, beta, U, X, R, out, s);
+    return launch_modal<float>(op, op->ks->km32[which], alpha, beta, U, X, R, out, s);
   }
   if (op->tensor) {
     const bool split = op->split[which];
