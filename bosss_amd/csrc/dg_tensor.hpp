@@ -421,12 +421,17 @@ template <int D, bool H> struct HandAdjoint<FormEuler<D, H>> : std::true_type {}
 template <class Form> struct IsHLLC : std::false_type {};
 template <int D> struct IsHLLC<FormEuler<D, true>> : std::true_type {};
 
-// Residual and JVP kernels of the Euler forms that use the volume table and the projected volume test
-// (QAcc).  Not the cell-split forms, whose workgroups would load the table for a quarter of the work
-// (p = 3 JVP, 12^3: 55 us without, 61 us with), nor the VJP kernels, whose registers are full (p = 3 fused,
-// 48^3: FP64 1640 / 1650 us, FP32 993 / 1642 us).
-template <class Form, bool SPLIT>
-constexpr bool euler_projects() { return HandAdjoint<Form>::value && !SPLIT; }
+// Euler kernels that use the volume table and the projected volume test (QAcc): the 3D residual except FP32
+// p = 2, and the FP64 p = 2 JVP.  Us without / with it, Rusanov and HLLC:
+//   residual 40^3   p = 2 FP64 133 / 124, 161 / 150   p = 3 FP64 398 / 387, 463 / 448   p = 3 FP32 246 / 218, 275 / 249
+//                   p = 2 FP32  87 /  91, 101 / 106   2D 512^2 110 / 123, 125 / 125
+//   JVP 25^3, 40^3  p = 2 FP64  60 /  56, 236 / 222 (Rusanov)
+//                   p = 2 FP32  42 /  45, 127 / 129   p = 3 FP32 104 / 110, 328 / 317 (Rusanov)   2D 512^2 247 / 255, 270 / 288
+// The p = 3 FP64 JVP has no registers left for it (48^3: 1260 / 1368), nor have the VJP kernels (p = 3 fused,
+// 48^3: FP64 1640 / 1650, FP32 993 / 1642).  The cell-split forms would load the table for a quarter of the
+// work (p = 3 JVP, 12^3: 55 / 61).
+template <class Form, int D, int P, typename Real, bool JVP, bool SPLIT>
+constexpr bool euler_projects() { return HandAdjoint<Form>::value && !SPLIT && D == 3 && (sizeof(Real) == 8 ? !JVP || P < 3 : !JVP && P == 3); }
 
 constexpr int TWAVES = 4;
 
@@ -493,7 +498,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   constexpr bool TAN = (MODE == MODE_JVP);
   constexpr int NARR = TAN ? 2 : 1;
   constexpr int STRIDE = NT | 1;
-  constexpr bool PROJ = euler_projects<Form, SPLIT>();   // volume table and projected volume test
+  constexpr bool PROJ = euler_projects<Form, D, P, Real, TAN, SPLIT>();   // volume table and projected volume test
   typedef typename std::conditional<TAN, Dual<1, Real>, Real>::type T;
 
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1074,7 +1079,7 @@ constexpr size_t kt_lds_bytes(int narrays) {
 template <class Form, int D, int P, int K1, typename Real>
 constexpr size_t kt_forward_lds_bytes(int narrays) {
   typedef TShape<D, P, K1> TS;
-  const size_t proj = HandAdjoint<Form>::value ? TS::VTAB + TWAVES * 16 * D * TS::NP : 0;   // volume table, q_fold staging
+  const size_t proj = euler_projects<Form, D, P, Real, false, false>() ? TS::VTAB + TWAVES * 16 * D * TS::NP : 0;   // volume table, q_fold staging
   return kt_lds_bytes<D, P, K1, Form::V, Real>(narrays) + (form_face_tables<Form, D>() * TS::FTAB + proj) * sizeof(Real);
 }
 
@@ -1380,8 +1385,7 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   Real* tab = reinterpret_cast<Real*>(smem_raw);
   Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * NSLOT * 64;
   for (int i = threadIdx.x; i < TS::TAB; i += blockDim.x) tab[i] = a.tab[i];
-  // FP64 p = 3 has no registers left for it (48^3: 1260 us without, 1368 us with, spilling)
-  constexpr bool PROJ = euler_projects<Form, SPLIT>() && (sizeof(Real) == 4 || P < 3);
+  constexpr bool PROJ = euler_projects<Form, D, P, Real, true, SPLIT>();
   if (PROJ) vt_load<TS>(ft, a.tab);   // the volume table first; the face table takes its place
   else ft_load<TS>(ft, a.tab);
   __syncthreads();
