@@ -494,16 +494,21 @@ static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks,
 // Whether the cell-split form of a kernel is taken.  A CU works through w = ceil(J / 64 / CUs) groups
 // of 64 cells or w4 = ceil(J / 16 / CUs) groups of 16, and a group of 16 takes `turn` of a group of 64:
 // a quarter and what a workgroup does once whatever its cells (tables into LDS, metrics, the sum of
-// the parts), which weighs more the less there is to do.  HLLC, us without / with the split form:
-//   p = 3 JVP       5^3 171 / 53, 20^3 182 / 117, 25^3 195 / 228, 31 x 29 x 37 548 / 491, 48^3 1260 / 1440
-//   p = 3 fused     5^3 227 / 70, 20^3 240 / 155, 25^3 256 / 300, 31 x 29 x 37 712 / 644, 48^3 1632 / 1888
-//   p = 3 residual  5^3 101 / 36, 20^3 108 /  77, 25^3 118 / 150, 31 x 29 x 37 335 / 331, 48^3  775 / 1033
-//   p = 2 JVP       5^3  69 / 27, 20^3  75 /  58, 25^3  82 / 111, 31 x 29 x 37 228 / 242, 48^3  537 /  709
+// the parts), which weighs more the less there is to do.  Us without / with the split form, on both sides of the line
+// (w, w4; cells), Rusanov, HLLC; it lies where no form and no precision loses:
+//                                FP64                          FP32
+//   p = 3 JVP       1, 3  23^3   154 / 143, 181 / 163          101 /  80, 124 / 103
+//                   3, 9  33.8 k 449 / 414, 531 / 474          250 / 219, 301 / 274
+//                   1, 4  25^3   157 / 186, 182 / 214          102 / 103, 126 / 128
+//   p = 3 residual  2, 5  18.3 k 181 / 163, 212 / 183          102 /  98, 117 / 107
+//                   2, 6  29^3   185 / 206, 215 / 227          108 / 118, 123 / 130
+//   p = 2 JVP       1, 2  20^3    54 /  45,  68 /  53           41 /  23,  53 /  28
+//                   1, 3  23^3    55 /  65,  68 /  78           41 /  35,  53 /  42
 // BOSSS_HIP_SPLIT=0 or 1 decides instead.
 static bool split_pays(int J, int num_cu, int D, int P, bool residual) {
   if (const char* x = std::getenv("BOSSS_HIP_SPLIT")) return x[0] == '1';
   // 2D: one volume tile, so a group of 16 takes more than half of a group of 64 (fused 80 x 80: 22 / 25 us)
-  const double turn = D == 2 ? 0.51 : P == 3 ? (residual ? 0.325 : 0.31) : 0.345;
+  const double turn = D == 2 ? 0.51 : P == 3 && !residual ? 0.31 : 0.345;
   const int w = ((J + 16 * TWAVES - 1) / (16 * TWAVES) + num_cu - 1) / num_cu, w4 = ((J + 15) / 16 + num_cu - 1) / num_cu;
   return turn * w4 < w;
 }
