@@ -49,12 +49,7 @@ struct TShape {
   static constexpr int TV = (KV + 15) / 16, TE = (KE + 15) / 16;
   static constexpr int NK = (N + 3) / 4, MT = (N + 15) / 16;
   static constexpr int O_L = 0, O_DL = (P + 1) * K2, O_W = 2 * (P + 1) * K2, O_CODE = O_W + K1;
-  // Derivative terms of mode m at O_DT + m * DT: d phi_m / d xi_e = c_e phi_(i_e) (+ c_3 phi_0 along the
-  // axis of a pure cubic): D + 1 slots (e * NP + i_e, the cubic's last), their coefficients, and what
-  // rounding took from these.  All modes i are of degree < P, the first NP.
-  static constexpr int NP = tdeg_count(D, P - 1), DT = 3 * (D + 1), O_DT = O_CODE + N;
-  static_assert(P <= 3, "one second derivative term per mode");
-  static constexpr int TAB = O_DT + N * DT;  // elements (Real) of the 1D table block
+  static constexpr int TAB = O_CODE + N;     // elements (Real) of the 1D table block
   // Face trace table FT[f][node][m] = phi_m at node `node` of face f, stored after the 1D block
   // in global memory: FROWS rows per face (whole 16-node tiles; the padding rows node >= KE hold
   // node 0's values, so a trace evaluated at them is a valid state), FS Real per row (modes
@@ -66,7 +61,12 @@ struct TShape {
   static constexpr int NFTAB = 1 + D;
   // Volume table phi_m at the volume nodes, rows and padding as in the face tables, after them.
   static constexpr int VTAB = TV * 16 * FS, O_VT = TAB + NFTAB * FTAB;
-  static_assert(VTAB <= FTAB, "the JVP and VJP kernels keep the volume table where the face table goes later");
+  // Derivative terms of mode m at m * DT behind it: d phi_m / d xi_e = c_e phi_(i_e) (+ c_3 phi_0 along the
+  // axis of a pure cubic): D + 1 slots (e * NP + i_e, the cubic's last), their coefficients, and what
+  // rounding took from these.  All modes i are of degree < P, the first NP.
+  static constexpr int NP = tdeg_count(D, P - 1), DT = 3 * (D + 1), O_DT = O_VT + VTAB, SIZE = O_DT + N * DT;
+  static_assert(P <= 3, "one second derivative term per mode");
+  static_assert(VTAB + N * DT <= FTAB, "the JVP kernel keeps the volume table and its terms where the face table goes later");
 };
 
 // Per-axis 1D indices of a node: volume node kv = (i*K1 + j)*K1 + k has x = k, y = j, z = i
@@ -269,9 +269,10 @@ __device__ __forceinline__ void t_test_ft(const Real* nrow, const FtCols<TS, Rea
   }
 }
 
+// Volume table and derivative terms.
 template <class TS, typename Real>
 __device__ __forceinline__ void vt_load(Real* vt, const Real* gtab) {
-  for (int i = threadIdx.x; i < TS::VTAB; i += blockDim.x) vt[i] = gtab[TS::O_VT + i];
+  for (int i = threadIdx.x; i < TS::VTAB + TS::N * TS::DT; i += blockDim.x) vt[i] = gtab[TS::O_VT + i];
 }
 
 // Volume test of the Euler forms, sum_e sum_k d_e phi_m g_e, by projection: d_e phi_m is a combination of
@@ -316,9 +317,9 @@ struct QAcc {
   }
 };
 
-// racc[v][m] += sum_e D_e[m][n] Q_e,n through `stage` (16 D NP Real of this wavefront's own).
+// racc[v][m] += sum_e D_e[m][n] Q_e,n through `stage` (16 D NP Real of this wavefront's own); terms: the derivative terms.
 template <class TS, typename Real, int V>
-__device__ __forceinline__ void q_fold(const Real* tab, Real* stage, int col, int grp, const QAcc<TS, Real, V>& q, TAcc<TS, Real, V>& racc) {
+__device__ __forceinline__ void q_fold(const Real* terms, Real* stage, int col, int grp, const QAcc<TS, Real, V>& q, TAcc<TS, Real, V>& racc) {
   typedef QAcc<TS, Real, V> Q;
 #pragma unroll
   for (int v = 0; v < V; v++) {
@@ -339,7 +340,7 @@ __device__ __forceinline__ void q_fold(const Real* tab, Real* stage, int col, in
       }
     __builtin_amdgcn_wave_barrier();
     racc.add(v, grp, [&](int m) {
-      const Real* d = tab + TS::O_DT + m * TS::DT;
+      const Real* d = terms + m * TS::DT;
       constexpr int NT = TS::P == 3 ? TS::D + 1 : TS::D;
       Real s = Real(0), x[NT];
 #pragma unroll
@@ -440,15 +441,14 @@ constexpr int TWAVES = 4;
 // a contiguous share of the face tiles (all faces of the cell, TE tiles each), and the partial results
 // are added through LDS in wavefront order.  The work unit is a quarter as long, for grids whose groups of
 // 64 cells leave CUs idle (split_pays).
-template <class TS>
+template <class TS, bool SPLIT>
 struct FaceShare {
   int lo, hi;   // face tiles f * TE + t of this wavefront
-  __device__ __forceinline__ FaceShare(bool split, int wave)
-      : lo(split ? wave * TS::NF * TS::TE / TWAVES : 0), hi(split ? (wave + 1) * TS::NF * TS::TE / TWAVES : TS::NF * TS::TE) {}
-  __device__ __forceinline__ int f0() const { return lo / TS::TE; }
-  __device__ __forceinline__ int f1() const { return (hi + TS::TE - 1) / TS::TE; }
-  __device__ __forceinline__ int t0(int f) const { return lo > f * TS::TE ? lo - f * TS::TE : 0; }
-  __device__ __forceinline__ int t1(int f) const { return hi < (f + 1) * TS::TE ? hi - f * TS::TE : TS::TE; }
+  __device__ __forceinline__ FaceShare(int wave) : lo(wave * TS::NF * TS::TE / TWAVES), hi((wave + 1) * TS::NF * TS::TE / TWAVES) {}
+  __device__ __forceinline__ int f0() const { return SPLIT ? lo / TS::TE : 0; }
+  __device__ __forceinline__ int f1() const { return SPLIT ? (hi + TS::TE - 1) / TS::TE : TS::NF; }
+  __device__ __forceinline__ int t0(int f) const { return SPLIT && lo > f * TS::TE ? lo - f * TS::TE : 0; }
+  __device__ __forceinline__ int t1(int f) const { return SPLIT && hi < (f + 1) * TS::TE ? hi - f * TS::TE : TS::TE; }
 };
 
 // This wavefront's accumulators to part[c * (NT | 1) + i] (cell c, entry i).
@@ -601,12 +601,12 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
     }
   }
 
-  if constexpr (PROJ) q_fold<TS, Real, V>(tab, vt + TS::VTAB + wave * (16 * D * TS::NP), col, grp, qacc, racc);
+  if constexpr (PROJ) q_fold<TS, Real, V>(vt + TS::VTAB, vt + TS::VTAB + N * TS::DT + wave * (16 * D * TS::NP), col, grp, qacc, racc);
 
   // ------------------------------------------------------------------- faces
   const Real pbd = Real(a.fp.penalty_base * a.fp.penalty_deg);
   const Real cj_own = Real(1.0 / a.lenscale[cj]);
-  const FaceShare<TS> share(SPLIT, wave);
+  const FaceShare<TS, SPLIT> share(wave);
   for (int f = share.f0(); f < share.f1(); f++) {
     const int nb_raw = a.cf.nb[(size_t)cj * NF + f];
     const int nb = valid ? nb_raw : -1;
@@ -1079,7 +1079,7 @@ constexpr size_t kt_lds_bytes(int narrays) {
 template <class Form, int D, int P, int K1, typename Real>
 constexpr size_t kt_forward_lds_bytes(int narrays) {
   typedef TShape<D, P, K1> TS;
-  const size_t proj = euler_projects<Form, D, P, Real, false, false>() ? TS::VTAB + TWAVES * 16 * D * TS::NP : 0;   // volume table, q_fold staging
+  const size_t proj = euler_projects<Form, D, P, Real, false, false>() ? TS::VTAB + TS::N * TS::DT + TWAVES * 16 * D * TS::NP : 0;   // volume table, terms, q_fold staging
   return kt_lds_bytes<D, P, K1, Form::V, Real>(narrays) + (form_face_tables<Form, D>() * TS::FTAB + proj) * sizeof(Real);
 }
 
@@ -1265,7 +1265,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
   }
 
   // ------------------------------------------------------------------- faces
-  const FaceShare<TS> share(SPLIT, wave);
+  const FaceShare<TS, SPLIT> share(wave);
   for (int f = share.f0(); f < share.f1(); f++) {
     const int nb_raw = a.cf.nb[(size_t)cj * NF + f];
     const int nb = valid ? nb_raw : -1;
@@ -1505,14 +1505,14 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   }
 
   if constexpr (PROJ) {
-    q_fold<TS, Real, V>(tab, buf, col, grp, qacc, racc);
+    q_fold<TS, Real, V>(vt + TS::VTAB, buf, col, grp, qacc, racc);
     __syncthreads();
     ft_load<TS>(ft, a.tab);
     __syncthreads();
   }
 
   // ------------------------------------------------------------------- faces
-  const FaceShare<TS> share(SPLIT, wave);
+  const FaceShare<TS, SPLIT> share(wave);
   for (int f = share.f0(); f < share.f1(); f++) {
     const int nb_raw = a.cf.nb[(size_t)cj * NF + f];
     const int nb = valid ? nb_raw : -1;

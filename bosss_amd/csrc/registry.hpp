@@ -104,7 +104,7 @@ KernelSet make_kernel_set(int kind) {
   constexpr int P = degree_from_modes(D, N);
   static_assert(tdeg_count(D, P) == N, "N must be a full total-degree basis");
   typedef TShape<D, P, K1> TSh;
-  k.P = P; k.ttab_size = TSh::O_VT + TSh::VTAB; k.t_o_dt = TSh::O_DT; k.t_o_vt = TSh::O_VT; k.t_vrows = TSh::TV * 16; k.t_np = TSh::NP; k.t_o_l = TSh::O_L; k.t_o_dl = TSh::O_DL; k.t_o_w = TSh::O_W; k.t_o_code = TSh::O_CODE;
+  k.P = P; k.ttab_size = TSh::SIZE; k.t_o_dt = TSh::O_DT; k.t_o_vt = TSh::O_VT; k.t_vrows = TSh::TV * 16; k.t_np = TSh::NP; k.t_o_l = TSh::O_L; k.t_o_dl = TSh::O_DL; k.t_o_w = TSh::O_W; k.t_o_code = TSh::O_CODE;
   k.t_k2 = TSh::K2;
   k.t_o_ft = TSh::TAB; k.t_frows = TSh::FROWS; k.t_fs = TSh::FS; k.t_ftab = TSh::FTAB;
   k.kt64[KernelSet::RES] = kt_forward<Form, D, P, K1, double, MODE_RES>;
