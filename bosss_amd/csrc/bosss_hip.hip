@@ -383,7 +383,7 @@ static void legendre_normalised(int P, double x, double* L, double* DL) {
 
 // Build the 1D table block of TShape and the face trace table after it, and check that the
 // uploaded tables are their tensor product.
-static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks, int K1, std::vector<double>& tab, double* maxdiff) {
+static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks, int K1, bool fp32, std::vector<double>& tab, double* maxdiff) {
   const int D = t->D, P = ks->P, K2 = ks->t_k2, N = t->N;
   tab.assign(ks->ttab_size, 0.0);
   if (t->Ke > ks->t_frows || ks->t_ftab != 2 * D * ks->t_frows * ks->t_fs || ks->t_o_ft + (1 + D) * ks->t_ftab != ks->t_o_vt ||
@@ -431,12 +431,14 @@ static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks,
       for (int d = 0; d < D; d++) cmp(val(q, ex[n], d), t->dphi[(k * N + n) * D + d]);
     }
   }
-  // derivative terms: ratios of the tables' values in the upper corner, a = num / den as hi + lo
+  // derivative terms: ratios of the kernels' table values in the upper corner (rounded to their precision), as
+  // hi + lo in that precision
+  auto rounded = [&](double v) { return fp32 ? (double)(float)v : v; };
   for (int n = 0; n < N; n++) {
     double* dt = &tab[ks->t_o_dt + (size_t)n * 3 * (D + 1)];
     const int up[3] = {K1 + 1, K1 + 1, K1 + 1};
     auto ratio = [&](int slot, int index, double num, double den) {
-      const double hi = num / den;
+      const double hi = rounded(num / den);
       dt[slot] = index;
       dt[D + 1 + slot] = hi;
       dt[2 * (D + 1) + slot] = std::fma(-hi, den, num) / den;
@@ -447,10 +449,10 @@ static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks,
       const int i = (int)(std::find(ex.begin(), ex.end(), ex[n] - (1 << (4 * e))) - ex.begin());
       if (i >= ks->t_np) return false;
       if (a < 3) {
-        ratio(e, e * ks->t_np + i, val(up, ex[n], e), val(up, ex[i], -1));
+        ratio(e, e * ks->t_np + i, rounded(val(up, ex[n], e)), rounded(val(up, ex[i], -1)));
       } else {               // a pure cubic: its share of phi_0 integrates to the difference of its traces
-        ratio(D, e * ks->t_np, val(up, ex[n], -1), val(up, ex[0], -1));
-        ratio(e, e * ks->t_np + i, val(up, ex[n], e) - val(up, ex[n], -1), val(up, ex[i], -1));
+        ratio(D, e * ks->t_np, rounded(val(up, ex[n], -1)), rounded(val(up, ex[0], -1)));
+        ratio(e, e * ks->t_np + i, rounded(val(up, ex[n], e)) - rounded(val(up, ex[n], -1)), rounded(val(up, ex[i], -1)));
       }
     }
   }
@@ -563,7 +565,7 @@ int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tabl
     std::vector<double> tab;
     double md = 0;
     const char* force_generic = std::getenv("BOSSS_HIP_GENERIC_TABLES");
-    op->tensor = ks->kt64[KernelSet::RES] && !(force_generic && force_generic[0] == '1') && build_tensor_tables(t, ks, K1, tab, &md);
+    op->tensor = ks->kt64[KernelSet::RES] && !(force_generic && force_generic[0] == '1') && build_tensor_tables(t, ks, K1, precision == BOSSS_FP32, tab, &md);
     op->ttab = nullptr;
     if (op->tensor) {
       if (precision == BOSSS_FP64) {

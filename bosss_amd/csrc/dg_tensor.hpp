@@ -279,12 +279,13 @@ __device__ __forceinline__ void vt_load(Real* vt, const Real* gtab) {
 // the NP modes of degree < P, so the nodes are contracted with those alone,
 //     Q_e,n = sum_k phi_n(k) g_e(k)       (n < NP: 10 of 20 modes at p = 3, 4 of 10 at p = 2),
 // and R_m = sum_e D_e[m][n] Q_e,n once per cell (q_fold).  A constant flux has to cancel between volume
-// and faces: D is the ratio of the rounded tables, with its own rounding error beside it (without: p = 2
-// residuals up to 24 % further from 64-bit exact).  The three directions share one operand, a
+// and faces: D is the ratio of the tables as rounded to Real, with its own rounding error beside it (FP64 p = 2
+// residuals without: up to 24 % further from 64-bit exact; FP32 p = 3, constant states: volume and faces differ by
+// 1.1e-7 of the faces on average with coefficients rounded once, by 4e-8 so).  The three directions share one operand, a
 // volume-table read, where the derivative tables took three 1D factors and a mode decode each; in
 // FP64 the rows go in fours (v_mfma_f64_4x4x4f64), 3 x 48 matrix cycles per variable and step instead of
-// 3 x 80 at p = 3, 3 x 16 instead of 3 x 64 at p = 2.  HLLC residual at 48^3: p = 3 FP32 468 -> 432 us,
-// FP64 777 -> 763 us, p = 2 279 -> 259 us; JVP p = 2 535 -> 510 us, p = 3 FP32 703 -> 689 us.
+// 3 x 80 at p = 3, 3 x 16 instead of 3 x 64 at p = 2.  HLLC residual at 48^3: p = 3 FP32 466 -> 427 us,
+// FP64 797 -> 766 us, p = 2 273 -> 254 us; JVP p = 2 508 -> 481 us.  Where it is used: euler_projects.
 template <class TS, typename Real, int V>
 struct QAcc {
   typedef typename MM<Real>::acc acc_t;
