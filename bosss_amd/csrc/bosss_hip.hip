@@ -686,8 +686,7 @@ static int launch_modal(const bosss_op* op, void (*k)(MArgs<Real>), double alpha
 static int launch(bosss_op* op, int which, double alpha, double beta, const void* U, const void* X, void* R, void* out, hipStream_t s,
                   int own_only = 0) {
   HIPCHK(hipSetDevice(op->ctx->device));
-  // Linear scalar forms on axis-aligned cells: the modal kernels (own_only probes of these forms
-  // do not come here, their diagonal blocks are assembled directly).
+  // Linear scalar forms on axis-aligned cells: the modal kernels, except for own_only probes.
   if (op->axis_nb && !own_only) {
     if (op->precision == BOSSS_FP64) return launch_modal<double>(op, op->ks->km64[which], alpha, beta, U, X, R, out, s);
     return launch_modal<float>(op, op->ks->km32[which], alpha, beta, U, X, R, out, s);
@@ -1000,6 +999,17 @@ static int ensure_matrix_setup(bosss_op* op) {
   return BOSSS_OK;
 }
 
+// A direct form whose tables or arrays are not made yet (its first call allocates them) does not run under
+// stream capture: there the probes do, on staging vectors that an earlier call has made.
+static int can_prepare(hipStream_t s, bool prepared, bool* direct) {
+  *direct = prepared;
+  if (prepared) return BOSSS_OK;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(s, &cs));
+  *direct = cs == hipStreamCaptureStatusNone;
+  return BOSSS_OK;
+}
+
 // Direct assembly of the linear forms (assemble_linear.hip): blocks of S slots per row, S = 1 the
 // diagonal alone.  The coefficient array is per operator and written by every call.
 static int assemble_linear(bosss_op* op, int S, double alpha, double beta, double shift, int transposed, double* blocks, hipStream_t s) {
@@ -1143,7 +1153,11 @@ int bosss_hip_op_assemble_dev(bosss_op* op, const double* U, double alpha, doubl
   // Linear forms: the blocks directly, unless a row reaches one cell across several faces (a
   // periodic direction of one or two cells), whose blocks add up in one slot: those rows, and the
   // Euler forms, go through the coloured probes.
-  if (!op->lin_host.empty() && !op->merged_slots) return assemble_linear(op, S, alpha, beta, 0.0, 0, blocks, s);
+  if (!op->lin_host.empty() && !op->merged_slots) {
+    bool direct;
+    if ((rc = can_prepare(s, op->d_lincoef, &direct))) return rc;
+    if (direct) return assemble_linear(op, S, alpha, beta, 0.0, 0, blocks, s);
+  }
   if ((rc = ensure_staging(op))) return rc;
   for (int k = 0; k < op->ncolors; k++)
     for (int q = 0; q < Nt; q++) {
@@ -1161,10 +1175,14 @@ int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, doub
   int rc;
   HIPCHK(hipSetDevice(op->ctx->device));
   hipStream_t s = (hipStream_t)stream;
-  if (!op->lin_host.empty()) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
+  const bool linear = !op->lin_host.empty();
+  bool direct;
+  if ((rc = can_prepare(s, linear ? op->d_lincoef : op->d_ebreal, &direct))) return rc;
+  if (linear && direct) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
   // Euler forms on tensor tables: directly, unless no kernel is built for them (2D); those and operators
   // on general tables go through the probes (20^3, p = 3: 17.4 ms by 100 probes, 1.18 ms directly).
-  if (op->tensor && (rc = euler_blocks(op, U, alpha, shift, (int)(transposed != 0), blocks, s)) != BOSSS_ERR_UNSUPPORTED) return rc;
+  if (op->tensor && !linear && direct && (rc = euler_blocks(op, U, alpha, shift, (int)(transposed != 0), blocks, s)) != BOSSS_ERR_UNSUPPORTED)
+    return rc;
   if ((rc = ensure_staging(op))) return rc;
   const int J = op->grid->J, Nt = op->V * op->N;
   const size_t n = (size_t)J * Nt;
