@@ -192,10 +192,6 @@ __device__ __forceinline__ void tile_store(const double (&a)[RA][RA], double* __
   }
 }
 
-// Waves per SIMD the register-tile kernel is compiled for: the column steps are latency bound.
-template <int RA>
-constexpr int lu_tile_waves() { return RA == 7 ? 3 : 1; }
-
 // Blocks of 21..16 RA DOF (the 100-DOF cell blocks of p = 3 Euler, up to 128): one workgroup of
 // 256 threads per block, the whole block in registers.  Thread (tc, tr) = (tid >> 4, tid & 15)
 // holds rows tr + 16 x and columns tc + 16 y (x, y < RA), in the block's original row order:
@@ -209,7 +205,7 @@ constexpr int lu_tile_waves() { return RA == 7 ? 3 : 1; }
 // Register columns and rows are picked with wavefront-uniform branches, so no register array is
 // indexed dynamically.
 template <int RA>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lu_tile_waves<RA>()))) k_block_lu_tile(int nblk, int nmax, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
+__global__ void __launch_bounds__(256) k_block_lu_tile(int nblk, int nmax, const int32_t* __restrict__ nsz, const int64_t* __restrict__ off,
                                                        double* __restrict__ A, int32_t* __restrict__ ipiv,
                                                        const int64_t* __restrict__ pivoff, int32_t* __restrict__ info) {
   __shared__ TileLDS<RA> L;

@@ -1025,20 +1025,14 @@ static int assemble_linear(bosss_op* op, int S, double alpha, double beta, doubl
   return BOSSS_OK;
 }
 
-// Diagonal blocks of the Euler forms from moments of their flux Jacobians (euler_blocks.hip);
-// BOSSS_ERR_UNSUPPORTED where no such kernel is built.
+// Diagonal blocks of the Euler forms from moments of their flux Jacobians (euler_blocks.hip).
 static int euler_blocks(bosss_op* op, const void* U, double alpha, double shift, int transposed, double* blocks, hipStream_t s) {
   const bosss_grid* g = op->grid;
-  const int P = op->ks->P;
-  // 3D alone: the 24 columns of the 2D p = 2 blocks cost little by probing, and by moments they measured
-  // 12 % further from 64-bit exact (7.1e-16 against 6.3e-16; 3D p = 2 8.5e-16 against 9.0e-16, p = 3
-  // 1.4e-15 against 1.7e-15)
-  if (op->D != 3) return BOSSS_ERR_UNSUPPORTED;
   if (!op->d_ebreal) {
     std::vector<double> x, w;
     gauss_legendre(op->K1, x, w);
     EulerBlockTables t;
-    euler_block_tables(op->D, P, op->K1, x, t);
+    euler_block_tables(op->ks->P, op->K1, x, t);
     int rc;
     if ((!op->d_ebints && (rc = upload(&op->d_ebints, t.ints.data(), t.ints.size()))) ||
         (rc = upload(&op->d_ebreal, t.real.data(), t.real.size())))
@@ -1050,8 +1044,7 @@ static int euler_blocks(bosss_op* op, const void* U, double alpha, double shift,
   for (int f = 0; f < 6; f++) a.cf.pair[f] = g->pair[f];
   a.fp = op->fp; a.real = op->d_ebreal; a.ints = op->d_ebints; a.U = U;
   a.alpha = alpha; a.shift = shift; a.transposed = transposed; a.blocks = blocks;
-  if (!launch_euler_blocks(op->kind == BOSSS_FORM_EULER_HLLC, op->D, P, op->K1, op->precision == BOSSS_FP32, op->ctx->num_cu, a, s))
-    return BOSSS_ERR_UNSUPPORTED;
+  launch_euler_blocks(op->kind == BOSSS_FORM_EULER_HLLC, op->ks->P, op->precision == BOSSS_FP32, op->ctx->num_cu, a, s);
   HIPCHK(hipGetLastError());
   return BOSSS_OK;
 }
@@ -1175,14 +1168,16 @@ int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, doub
   int rc;
   HIPCHK(hipSetDevice(op->ctx->device));
   hipStream_t s = (hipStream_t)stream;
+  // Linear forms, and the 3D Euler forms on tensor tables, directly; 2D Euler and Euler on general tables by
+  // probes (20^3, p = 3: 17.4 ms by 100 probes, 1.18 ms directly).
   const bool linear = !op->lin_host.empty();
-  bool direct;
-  if ((rc = can_prepare(s, linear ? op->d_lincoef : op->d_ebreal, &direct))) return rc;
-  if (linear && direct) return assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s);
-  // Euler forms on tensor tables: directly, unless no kernel is built for them (2D); those and operators
-  // on general tables go through the probes (20^3, p = 3: 17.4 ms by 100 probes, 1.18 ms directly).
-  if (op->tensor && !linear && direct && (rc = euler_blocks(op, U, alpha, shift, (int)(transposed != 0), blocks, s)) != BOSSS_ERR_UNSUPPORTED)
-    return rc;
+  if (linear || (op->tensor && has_euler_blocks(op->D, op->ks->P, op->K1))) {
+    bool direct;
+    if ((rc = can_prepare(s, linear ? op->d_lincoef : op->d_ebreal, &direct))) return rc;
+    if (direct)
+      return linear ? assemble_linear(op, 1, alpha, 0.0, shift, (int)(transposed != 0), blocks, s)
+                    : euler_blocks(op, U, alpha, shift, (int)(transposed != 0), blocks, s);
+  }
   if ((rc = ensure_staging(op))) return rc;
   const int J = op->grid->J, Nt = op->V * op->N;
   const size_t n = (size_t)J * Nt;

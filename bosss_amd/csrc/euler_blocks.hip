@@ -1,7 +1,7 @@
 // Diagonal blocks of the Euler Jacobian, dR_j/dU_j + shift I per cell, from moments of the pointwise
-// flux Jacobians.
+// flux Jacobians; 3D alone.
 //
-// With A_e(x) = detJ sc^2 sum_d invJ[e][d] dF_d/dU the 5 x 5 Jacobian at a node (4 x 4 in 2D), the
+// With A_e(x) = detJ sc^2 sum_d invJ[e][d] dF_d/dU the 5 x 5 Jacobian at a node, the
 // volume part of entry ((v, n), (w, m)) is sum_e sum_k w_k d_e phi_n A_e,vw phi_m.  d_e phi_n is a short
 // combination of modes of degree < p, and the product of two modes a short combination of Legendre
 // products of degree <= 2 p - 1 (one to four terms), so the entry is a short combination of the moments
@@ -30,11 +30,11 @@
 
 namespace bosss {
 
-template <int D_, int P_, int K1_>
+template <int P_, int K1_>
 struct EB {
-  static constexpr int D = D_, P = P_, K1 = K1_, K2 = K1 + 2, V = D + 2, N = tdeg_count(D, P), NT = V * N;
+  static constexpr int D = 3, P = P_, K1 = K1_, K2 = K1 + 2, V = D + 2, N = tdeg_count(D, P), NT = V * N;
   static constexpr int KV = ipow(K1, D), KE = ipow(K1, D - 1);
-  static constexpr int LV = tdeg_count(D, 2 * P - 1), LF = D == 3 ? tdeg_count(2, 2 * P) : 2 * P + 1;   // moments per pair
+  static constexpr int LV = tdeg_count(D, 2 * P - 1), LF = tdeg_count(2, 2 * P);   // moments per pair
   static constexpr int KSV = (KV + 3) / 4, KSF = (KE + 3) / 4;      // MFMA k-steps
   static constexpr int RV = (LV + 15) / 16, RF = (LF + 15) / 16;    // 16-row tiles
   static constexpr int VV = V * V, CT = (VV + 15) / 16;             // Jacobian entries, 16-column tiles
@@ -70,14 +70,9 @@ __device__ __forceinline__ double node_value(const double* L, const double* u, c
 #pragma unroll
     for (int a = 0; a <= deg; a++) {
       double t = 0.0;
-      if (E::D == 3) {
 #pragma unroll
-        for (int b = 0; b <= deg - a; b++) {
-          t += u[n] * (L[b * E::K2 + q[1]] * L[(deg - a - b) * E::K2 + q[2]]);
-          n++;
-        }
-      } else {
-        t = u[n] * L[(deg - a) * E::K2 + q[1]];
+      for (int b = 0; b <= deg - a; b++) {
+        t += u[n] * (L[b * E::K2 + q[1]] * L[(deg - a - b) * E::K2 + q[2]]);
         n++;
       }
       s[a] += t;
@@ -113,11 +108,11 @@ __device__ __forceinline__ void add_terms(const EulerBlockArgs& a, int phase, in
   }
 }
 
-template <class Form, int D, int P, int K1, typename Real>
+template <class Form, int P, int K1, typename Real>
 __global__ void __launch_bounds__(256, 2) k_euler_blocks(EulerBlockArgs a) {
-  typedef EB<D, P, K1> E;
+  typedef EB<P, K1> E;
   typedef Dual<1, double> T;
-  constexpr int V = E::V, N = E::N, NT = E::NT, VV = E::VV, KV = E::KV, KE = E::KE, CTW = E::WIDE ? E::CT : 1;
+  constexpr int D = E::D, V = E::V, N = E::N, NT = E::NT, VV = E::VV, KV = E::KV, KE = E::KE, CTW = E::WIDE ? E::CT : 1;
   extern __shared__ __align__(16) double smem[];
   double* L = smem;
   double* uo = L + (P + 1) * E::K2;      // own coefficients, then both neighbours of a direction
@@ -326,7 +321,6 @@ static std::vector<std::vector<int>> total_degree(int D, int p) {   // by degree
   std::vector<std::vector<int>> e;
   for (int deg = 0; deg <= p; deg++)
     for (int a = 0; a <= deg; a++) {
-      if (D == 1) { if (a == deg) e.push_back({a, 0, 0}); continue; }
       for (int b = 0; b <= deg - a; b++) {
         if (D == 2 && a + b != deg) continue;
         e.push_back({a, b, D == 3 ? deg - a - b : 0});
@@ -342,8 +336,8 @@ static ext legendre(int n, ext x) {   // normalised
   return std::sqrt(n + 0.5L) * p1;
 }
 
-void euler_block_tables(int D, int P, int K1, const std::vector<double>& nodes, EulerBlockTables& t) {
-  const int K2 = K1 + 2;
+void euler_block_tables(int P, int K1, const std::vector<double>& nodes, EulerBlockTables& t) {
+  const int D = 3, K2 = K1 + 2;
   const auto modes = total_degree(D, P), vol = total_degree(D, 2 * P - 1), face = total_degree(D - 1, 2 * P);
   const int N = (int)modes.size(), LV = (int)vol.size(), LF = (int)face.size(), V = D + 2, MS = (V * V + 1) & ~1;
   int KE = 1;
@@ -401,11 +395,11 @@ void euler_block_tables(int D, int P, int K1, const std::vector<double>& nodes, 
           }
         }
         // face coordinates (s0, s1): the tangential axes in the order the node index runs over them
-        const int s0 = D == 2 ? 1 - e : (e == 0 ? 2 : 0), s1 = D == 2 ? -1 : (e == 2 ? 1 : (e == 0 ? 1 : 2));
+        const int s0 = e == 0 ? 2 : 0, s1 = e == 2 ? 1 : (e == 0 ? 1 : 2);
         const int odd = (modes[n][e] + modes[m][e]) & 1;
         for (int l = 0; l < LF; l++) {
           ext c = norm * std::sqrt((modes[n][e] + 0.5L) * (modes[m][e] + 0.5L)) * legendre_product(modes[n][s0], modes[m][s0], face[l][0]);
-          if (D == 3) c *= legendre_product(modes[n][s1], modes[m][s1], face[l][1]);
+          c *= legendre_product(modes[n][s1], modes[m][s1], face[l][1]);
           add(terms[D + e][n * N + m], odd * LF + l, c);
         }
       }
@@ -440,25 +434,25 @@ void euler_block_tables(int D, int P, int K1, const std::vector<double>& nodes, 
   t.ints.insert(t.ints.end(), idx.begin(), idx.end());
 }
 
-template <class Form, int D, int P, int K1>
+template <class Form, int P, int K1>
 static void launch_blocks(bool fp32, int num_cu, const EulerBlockArgs& a, hipStream_t s) {
-  typedef EB<D, P, K1> E;
+  typedef EB<P, K1> E;
   const size_t lds = (size_t)(E::LDS + 2) * sizeof(double);
   const dim3 grid((unsigned)std::min(a.J, 2 * num_cu));   // two workgroups per CU (registers), each walking its cells
-  if (fp32) hipLaunchKernelGGL((k_euler_blocks<Form, D, P, K1, float>), grid, dim3(256), lds, s, a);
-  else hipLaunchKernelGGL((k_euler_blocks<Form, D, P, K1, double>), grid, dim3(256), lds, s, a);
+  if (fp32) hipLaunchKernelGGL((k_euler_blocks<Form, P, K1, float>), grid, dim3(256), lds, s, a);
+  else hipLaunchKernelGGL((k_euler_blocks<Form, P, K1, double>), grid, dim3(256), lds, s, a);
 }
-template <int D, int P, int K1>
+template <int P, int K1>
 static void launch_form(bool hllc, bool fp32, int num_cu, const EulerBlockArgs& a, hipStream_t s) {
-  if (hllc) launch_blocks<FormEuler<D, true>, D, P, K1>(fp32, num_cu, a, s);
-  else launch_blocks<FormEuler<D, false>, D, P, K1>(fp32, num_cu, a, s);
+  if (hllc) launch_blocks<FormEuler<3, true>, P, K1>(fp32, num_cu, a, s);
+  else launch_blocks<FormEuler<3, false>, P, K1>(fp32, num_cu, a, s);
 }
 
-bool launch_euler_blocks(bool hllc, int D, int P, int K1, bool fp32, int num_cu, const EulerBlockArgs& a, hipStream_t s) {
-  if (D == 3 && P == 2 && K1 == 4) launch_form<3, 2, 4>(hllc, fp32, num_cu, a, s);
-  else if (D == 3 && P == 3 && K1 == 5) launch_form<3, 3, 5>(hllc, fp32, num_cu, a, s);
-  else return false;
-  return true;
+bool has_euler_blocks(int D, int P, int K1) { return D == 3 && ((P == 2 && K1 == 4) || (P == 3 && K1 == 5)); }
+
+void launch_euler_blocks(bool hllc, int P, bool fp32, int num_cu, const EulerBlockArgs& a, hipStream_t s) {
+  if (P == 2) launch_form<2, 4>(hllc, fp32, num_cu, a, s);
+  else launch_form<3, 5>(hllc, fp32, num_cu, a, s);
 }
 
 }  // namespace bosss
