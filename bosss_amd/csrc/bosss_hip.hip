@@ -583,17 +583,20 @@ int bosss_hip_op_create(bosss_ctx* ctx, const bosss_grid* grid, const bosss_tabl
     add(t->vol_weights, Kv); add(t->phi, Kv * N); add(t->dphi, Kv * N * D);
     add(t->face_weights, Ke); add(t->trace, NF * Ke * N); add(t->dtrace, NF * Ke * N * D);
   }
-  if ((rc = ks->prepare()) != 0) { bosss_hip_op_destroy(op); return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc); }
-  if (op->tensor && (precision == BOSSS_FP64 ? (const void*)ks->km64[KernelSet::RES] : (const void*)ks->km32[KernelSet::RES])) {
-    if ((rc = axis_arrays(grid)) != BOSSS_OK) { bosss_hip_op_destroy(op); return rc; }
-    op->axis_real = grid->axis_real;
-    op->axis_nb = grid->axis_nb;
-  }
   if (op->tensor)
     for (int i = 0; i < KernelSet::NVARIANT; i++) {
       const void* part = precision == BOSSS_FP64 ? (const void*)ks->kts64[i] : (const void*)ks->kts32[i];
       if (part) op->split[i] = split_pays(grid->J, ctx->num_cu, t->D, ks->P, i == KernelSet::RES);
     }
+  if ((rc = ks->prepare(precision == BOSSS_FP32, op->tensor, op->split)) != 0) {
+    bosss_hip_op_destroy(op);
+    return fail(BOSSS_ERR_HIP, "kernel attribute setup failed (%d)", rc);
+  }
+  if (op->tensor && (precision == BOSSS_FP64 ? (const void*)ks->km64[KernelSet::RES] : (const void*)ks->km32[KernelSet::RES])) {
+    if ((rc = axis_arrays(grid)) != BOSSS_OK) { bosss_hip_op_destroy(op); return rc; }
+    op->axis_real = grid->axis_real;
+    op->axis_nb = grid->axis_nb;
+  }
   *out = op;
   return BOSSS_OK;
 }

@@ -24,14 +24,18 @@ const KernelSet* find_kernels(int kind, int D, int N, int K1, int precision) {
   return nullptr;
 }
 
-int KernelSet::prepare() const {
+int KernelSet::prepare(bool fp32, bool tensor, const bool* split) const {
   for (int i = 0; i < NVARIANT; i++) {
-    if (k64[i] && hipFuncSetAttribute((const void*)k64[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64) != hipSuccess) return 1;
-    if (k32[i] && hipFuncSetAttribute((const void*)k32[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds32) != hipSuccess) return 2;
-    if (kt64[i] && hipFuncSetAttribute((const void*)kt64[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds64[i]) != hipSuccess) return 3;
-    if (kts64[i] && hipFuncSetAttribute((const void*)kts64[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds64[i]) != hipSuccess) return 5;
-    if (kts32[i] && hipFuncSetAttribute((const void*)kts32[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds32[i]) != hipSuccess) return 6;
-    if (kt32[i] && hipFuncSetAttribute((const void*)kt32[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)ktlds32[i]) != hipSuccess) return 4;
+    const void* k;
+    size_t lds;
+    if (!tensor) {
+      k = fp32 ? (const void*)k32[i] : (const void*)k64[i];
+      lds = fp32 ? lds32 : lds64;
+    } else {
+      k = fp32 ? (const void*)(split[i] ? kts32 : kt32)[i] : (const void*)(split[i] ? kts64 : kt64)[i];
+      lds = fp32 ? ktlds32[i] : ktlds64[i];
+    }
+    if (k && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return 1 + i;
   }
   return 0;
 }

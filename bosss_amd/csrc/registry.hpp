@@ -31,7 +31,9 @@ struct KernelSet {
   // modal kernels (dg_modal.hpp) of the linear scalar forms on axis-aligned grids, or nullptr
   void (*km64[NVARIANT])(MArgs<double>);
   void (*km32[NVARIANT])(MArgs<float>);
-  int prepare() const;
+  // Allows the dynamic LDS of the kernels an operator launches (no others: the first use of a kernel loads its code
+  // object; the first Euler operator of a process takes 1.9 ms, 7.1 ms with every form of it).
+  int prepare(bool fp32, bool tensor, const bool* split) const;
 };
 
 constexpr int degree_from_modes(int D, int N) {
