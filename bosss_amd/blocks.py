@@ -21,7 +21,7 @@ class BlockBatch:
         import torch
         self.sizes = np.asarray(sizes, dtype=np.int32)
         if self.sizes.min() < 1 or self.sizes.max() > 4096:
-            raise ValueError("block sizes must be in 1..4096 (above 128: factored in global memory, no inverse)")
+            raise ValueError("block sizes must be in 1..4096 (above 128: no inverse)")
         n64 = self.sizes.astype(np.int64)
         off = np.zeros(len(n64), np.int64); off[1:] = np.cumsum(n64 * n64)[:-1]
         xoff = np.zeros(len(n64), np.int64); xoff[1:] = np.cumsum(n64)[:-1]
@@ -206,7 +206,7 @@ class Schwarz:
     parts: lists of cell indices; with overlap > 0 each part grows by that many layers of
     neighbouring cells (the matrix pattern's neighbours).  Init reads every part's dense
     block from the operator matrix in block-ELL layout (one gather) and factors all parts in
-    one batched launch (getrf semantics; parts above 128 DOF factor in global memory).
+    one batched call (getrf semantics).
     Solve(x, b, sweeps): per sweep, Res = b - M x, then x += sum_parts R_p^T A_p^-1 R_p Res,
     the corrections of overlapping cells summed in part order (no overlap scaling: the
     reference's default EnableOverlapScaling = false).

@@ -6,11 +6,11 @@
 // beaten); a zero pivot sets INFO = j+1 (1-based) and the factorisation continues.
 // Pivots are stored 1-based (ipiv).  Blocks up to 20 DOF keep their rows in registers
 // (several blocks per wavefront), 21..128 DOF one block per workgroup in registers,
-// larger ones (Schwarz blocks) go through global memory.
+// larger ones (Schwarz blocks) are blocked: panels in registers up to 1024 DOF where the
+// caller keeps the pivots, in global memory otherwise.
 //
-// All blocks of a batch are processed by one launch (blocks of different size
-// share the launch; each wave reads its own size), so a whole block-Jacobi set
-// of uneven XDG blocks (10x10 and 20x20) is one kernel.
+// Blocks of different size share a launch (each wave reads its own size), so a whole
+// block-Jacobi set of uneven XDG blocks (10x10 and 20x20) is one kernel.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -672,8 +672,8 @@ __global__ void __launch_bounds__(256) k_block_lu_rows(int nblk, int nmax, const
   if (ok && r == 0 && info) info[b] = inf;
 }
 
-// Blocks above LU_MAXN (the multi-cell blocks of Schwarz smoothers, up to LU_BIG_MAXN) factor in
-// place in global memory, blocked (see the blocked forms below); the pivot search is getf2's:
+// Blocks above LU_MAXN (the multi-cell blocks of Schwarz smoothers, up to LU_BIG_MAXN), pivots not kept or above
+// LU_REG_MAXN: in place in global memory, blocked (see the blocked forms below); the pivot search is getf2's:
 // the first row with the largest |a| in the column (workgroup argmax, ties to the smaller row).
 constexpr int LU_BIG_MAXN = 4096;
 // the two-launch-per-panel form takes over for blocks of at least LU_SPLIT_MINN when the batch
@@ -1197,7 +1197,8 @@ __global__ void __launch_bounds__(64) k_lu_first_zero(int nblk, int nmax, const 
 //
 // Bound: the 2 n dependent steps of the diagonal tiles, half of them with a division.  48 blocks of
 // 200..540 DOF: 1.67 ms by one wavefront per block walking the factor's columns in memory, 0.20 ms here;
-// 300 of 100 DOF 0.14 -> 0.08 ms.  Measured and not kept: lane partial sums of the rows (0.20 ms too, and
+// 300 of 128 DOF 0.135 -> 0.062 ms, 31000 of 10 DOF 88 -> 79 us, of 10 and 20 mixed 171 -> 119 us (the wide kernel's
+// workgroups that find a small block and return are within these).  Measured and not kept: lane partial sums of the rows (0.20 ms too, and
 // other rounding), the division by a Newton step on a reciprocal (0.23 ms).
 constexpr int SOLVE_SMALL = 128, SOLVE_T = 64, SOLVE_WAVES = 8;
 

@@ -19,8 +19,8 @@
 //
 // Bound: HBM and L2 traffic (own and 2D neighbour coefficients, one store), where the nodal kernels
 // of dg_tensor.hpp are bound by their dense contractions.  Upwind + SIP p = 3 residual at 64^3, FP64:
-// 522 us by the nodal kernel, 47 us here (84 MB of coefficients in and out, 31 MB of metrics); FP32
-// adjoint at 45 x 37 x 29: 65 -> 9.5 us, the cost of the call.  Measured and not kept: all faces
+// a call takes 522 us with the nodal kernel, 51 us here (the kernel 47; 84 MB of coefficients in and out, 31 MB of
+// metrics); FP32 adjoint at 45 x 37 x 29: 65 -> 11 us.  Measured and not kept: all faces
 // unrolled (448 registers, 60 us), neighbour coefficients gathered through an LDS tile (67 us: the
 // lane exchange of the cell indices costs more than the scattered lines), results stored without
 // the tile (55 us), three wavefronts per SIMD (100 us, spills).

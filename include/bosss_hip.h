@@ -160,12 +160,13 @@ int bosss_hip_op_assemble_dev(bosss_op* op, const double* U, double alpha, doubl
 /* Diagonal cell blocks of the Jacobian, for cell-block preconditioners (the blocks BlockJacobi.InitImpl
  * reads from the assembled matrix, BlockJacobi.cs:63-120, without assembling the off-diagonal ones):
  * blocks[j] <- alpha * dR_j/dU_j (U) + shift * I, row-major Nt x Nt (Nt = V*N), J blocks of FP64;
- * with transposed != 0 each block is stored transposed (column-major), which is how the probes
- * produce it (one column per probe, written contiguously): inverting those blocks in place gives
- * the transposed inverses that bosss_hip_block_gemv_uniform_dev applies.
- * Nt probing JVPs with the neighbour tangents taken as zero, in the operator's precision (U is
- * double for BOSSS_FP64, float for BOSSS_FP32; an FP32 operator gives FP32-accurate blocks, widened).
- * Works for every form, linear or not. */
+ * with transposed != 0 each block is stored transposed (column-major): inverting those blocks in
+ * place gives the transposed inverses that bosss_hip_block_gemv_uniform_dev applies.
+ * U is a state vector of the operator (double for BOSSS_FP64, float for BOSSS_FP32).  Linear forms and
+ * the 3D Euler forms on tensor tables form the blocks directly, in 64 bits whatever the precision; the
+ * first such call on an operator allocates.  The others, and a first call under stream capture (on staging
+ * vectors an earlier call has made), take Nt probing JVPs with the neighbour tangents zero, in the
+ * operator's precision. */
 int bosss_hip_op_diag_blocks_dev(bosss_op* op, const void* U, double alpha, double shift, int32_t transposed, double* blocks,
                                  void* stream);
 /* y <- alpha*A x + beta*y with A in the operator's block-ELL layout (BlockMsrMatrix.SpMV, BlockMsrMatrix.cs:2554) */
@@ -191,12 +192,13 @@ int bosss_hip_op_spmv_tiles(const bosss_op* op, int32_t* chosen, int32_t* ncand,
  *      4096 DOF, Schwarz.cs:827-915; above that the reference switches to PARDISO).
  *      Blocks are dense row-major at element offsets off[b], sizes n[b] <= nmax <= 4096:
  *      nmax <= 128 holds each block in registers (up to 20 DOF several blocks per
- *      wavefront, above that one 256-thread workgroup per block); larger nmax
- *      factors in place in global memory, blocked: getf2 on 32-column panels (the same
- *      pivots), the trailing update as a rank-32 product on the matrix units (one
- *      256-thread workgroup per block, or, for fewer than 256 blocks with nmax >= 512,
- *      two launches per panel with the trailing update over many workgroups; that form
- *      synchronises the stream before it returns).
+ *      wavefront, above that one 256-thread workgroup per block); larger nmax is blocked:
+ *      getf2 on 32-column panels (the same pivots), the trailing update as a rank-32 product
+ *      on the matrix units.  nmax <= 1024 with ipiv and at most 65535 blocks: panels in
+ *      registers, two launches per panel, no allocation, no synchronisation.  Otherwise in
+ *      place in global memory: one 256-thread workgroup per block, or, for fewer than 256
+ *      blocks with nmax >= 512, two launches per panel; that form allocates and synchronises
+ *      the stream before it returns.
  *      ipiv (1-based, LAPACK convention) at pivoff[b]; info[b] as DGETRF's INFO
  *      (0, or j+1 for the first zero pivot; -1 if n[b] exceeds nmax).  The inverse
  *      (want_inverse) needs nmax <= 128.  In
@@ -205,20 +207,20 @@ int bosss_hip_op_spmv_tiles(const bosss_op* op, int32_t* chosen, int32_t* ncand,
  *      want_inverse != 0 overwrites each block with its inverse (DGETRI's result, above
  *      20 DOF by in-place Gauss-Jordan with the same pivot rows), n <= 128; a singular
  *      block keeps its LU factors instead, with INFO set.
- *      All arrays are device memory; one launch covers the whole batch. ---- */
+ *      All arrays are device memory; one call covers the whole batch. ---- */
 int bosss_hip_block_lu_dev(bosss_ctx* ctx, int nblk, int32_t nmax, const int32_t* n, const int64_t* off, double* A,
                            int32_t* ipiv, const int64_t* pivoff, int32_t* info, int32_t want_inverse, void* stream);
 /* The same factorisation without allocating: no counterpart in the reference; for callers that
  * cannot allocate device memory (code under HIP graph capture, tight solver loops, hosts that
- * forbid hipMalloc).  Blocks above 128 DOF always use the split form (two launches per panel,
- * same pivots and factors as above) with its per-block status words in a fixed device
- * array of the library (8 KiB per device, held until the process ends), so at most 1024 such
- * blocks per call (BOSSS_ERR_ARG beyond); up to 128 DOF it is the register kernels above,
- * which need no scratch.  The call only queues work on `stream` and never synchronises.  Every call on one
- * device shares that array: calls that overlap on one device race. */
+ * forbid hipMalloc).  Up to 128 DOF, and up to 1024 DOF with ipiv, it is the register kernels above, which
+ * need no scratch; other blocks use two launches per panel (same pivots and factors) with the per-block
+ * status words in a fixed device array of the library (8 KiB per device, held until the process ends).  At
+ * most 1024 blocks per call above 128 DOF in either form (BOSSS_ERR_ARG beyond: one limit, whatever ipiv).
+ * The call only queues work on `stream` and never synchronises.  Calls that use the fixed array share it:
+ * those that overlap on one device race. */
 int bosss_hip_block_lu_noalloc_dev(bosss_ctx* ctx, int nblk, int32_t nmax, const int32_t* n, const int64_t* off, double* A,
                                    int32_t* ipiv, const int64_t* pivoff, int32_t* info, int32_t want_inverse, void* stream);
-/* x_b <- (LU_b)^-1 x_b  (DGETRS), x_b at element offset xoff[b] */
+/* x_b <- (LU_b)^-1 x_b  (DGETRS), x_b at element offset xoff[b]; any block size */
 int bosss_hip_block_solve_dev(bosss_ctx* ctx, int nblk, const int32_t* n, const int64_t* off, const double* LU,
                               const int32_t* ipiv, const int64_t* pivoff, const int64_t* xoff, double* x, void* stream);
 /* y_b <- alpha Ainv_b x_b + beta y_b  (block-diagonal apply of BlockJacobi.Solve, BlockJacobi.cs:148-197) */
