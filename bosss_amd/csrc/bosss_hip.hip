@@ -75,7 +75,7 @@ struct bosss_grid {
   mutable std::mutex axis_lock;
   mutable bool axis_known = false;
   mutable double* axis_real = nullptr;   // [D][J] invJ diagonal, [NF][J] sqrtg
-  mutable int* axis_nb = nullptr;        // [NF][J]
+  mutable int* axis_nb = nullptr;        // [NF][J], in the same allocation
 };
 
 struct bosss_op {
@@ -160,9 +160,9 @@ static int axis_arrays(const bosss_grid* G) {
   const size_t J = G->J, nreal = (size_t)(G->D + G->NF) * J, nnb = (size_t)G->NF * J;
   hipStream_t s = G->ctx->stream;
   double* real = nullptr;
-  int *anb = nullptr, skew = 0;
-  hipError_t e = hipMalloc((void**)&real, nreal * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void**)&anb, (nnb + 1) * sizeof(int));   // the flag behind the neighbours
+  int skew = 0;
+  hipError_t e = hipMalloc((void**)&real, nreal * sizeof(double) + (nnb + 1) * sizeof(int));
+  int* anb = reinterpret_cast<int*>(real + nreal);   // the neighbours, the flag behind them
   if (e == hipSuccess) e = hipMemsetAsync(anb + nnb, 0, sizeof(int), s);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_axis_arrays, dim3((unsigned)((J + 255) / 256)), dim3(256), 0, s, G->J, G->D, G->invJ, G->sqrtg, G->normal, G->nb,
@@ -173,7 +173,6 @@ static int axis_arrays(const bosss_grid* G) {
   if (e == hipSuccess) e = hipStreamSynchronize(s);   // any stream may read the arrays from here on
   if (e != hipSuccess || skew) {
     (void)hipFree(real);
-    (void)hipFree(anb);
     real = nullptr;
     anb = nullptr;
   }
@@ -316,7 +315,7 @@ int bosss_hip_grid_destroy(bosss_grid* g) {
   if (!g) return BOSSS_OK;
   (void)hipFree(g->detJ); (void)hipFree(g->invJ); (void)hipFree(g->scaling); (void)hipFree(g->lenscale);
   (void)hipFree(g->nb); (void)hipFree(g->sqrtg); (void)hipFree(g->normal);
-  (void)hipFree(g->axis_real); (void)hipFree(g->axis_nb);
+  (void)hipFree(g->axis_real);
   delete g;
   return BOSSS_OK;
 }
