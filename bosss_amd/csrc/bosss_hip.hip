@@ -386,7 +386,7 @@ static bool build_tensor_tables(const bosss_tables_desc* t, const KernelSet* ks,
   const int D = t->D, P = ks->P, K2 = ks->t_k2, N = t->N;
   tab.assign(ks->ttab_size, 0.0);
   if (t->Ke > ks->t_frows || ks->t_ftab != 2 * D * ks->t_frows * ks->t_fs || ks->t_o_ft + (1 + D) * ks->t_ftab != ks->t_o_vt ||
-      ks->t_o_vt + ks->t_vrows * ks->t_fs != ks->t_o_dt || ks->t_o_dt + 3 * (D + 1) * N != ks->ttab_size || t->Kv > ks->t_vrows)
+      ks->t_o_dt + 3 * (D + 1) * N != ks->t_o_ft || ks->t_o_vt + ks->t_vrows * ks->t_fs != ks->ttab_size || t->Kv > ks->t_vrows)
     return false;
   std::vector<double> x, w;
   gauss_legendre(K1, x, w);

@@ -50,7 +50,14 @@ struct TShape {
   static constexpr int NK = (N + 3) / 4, MT = (N + 15) / 16;
   static constexpr int O_L = 0, O_DL = (P + 1) * K2, O_W = 2 * (P + 1) * K2, O_CODE = O_W + K1;
   static constexpr int TAB = O_CODE + N;     // elements (Real) of the 1D table block
-  // Face trace table FT[f][node][m] = phi_m at node `node` of face f, stored after the 1D block
+  // Derivative terms of mode m at O_DT + m * DT: d phi_m / d xi_e = c_e phi_(i_e) (+ c_3 phi_0 along the
+  // axis of a pure cubic): D + 1 slots (e * NP + i_e, the cubic's last), their coefficients, and what
+  // rounding took from these.  All modes i are of degree < P, the first NP.
+  static constexpr int NP = tdeg_count(D, P - 1), DT = 3 * (D + 1), O_DT = TAB, O_FT = O_DT + N * DT;
+  static_assert(P <= 3, "one second derivative term per mode");
+  // elements of a kernel's LDS copy: with the terms if it projects (a multiple of 2, for what follows)
+  static constexpr int tab_lds(bool proj) { return ((proj ? O_FT : TAB) + 1) & ~1; }
+  // Face trace table FT[f][node][m] = phi_m at node `node` of face f, stored after these
   // in global memory: FROWS rows per face (whole 16-node tiles; the padding rows node >= KE hold
   // node 0's values, so a trace evaluated at them is a valid state), FS Real per row (modes
   // m >= N and the columns FZERO, FZERO + 1 are zero).  FS = 4 NK + 2 keeps the LDS reads of
@@ -60,13 +67,8 @@ struct TShape {
   // 1 + D face tables in this layout follow each other: phi_m, then d phi_m / d xi_e, e < D.
   static constexpr int NFTAB = 1 + D;
   // Volume table phi_m at the volume nodes, rows and padding as in the face tables, after them.
-  static constexpr int VTAB = TV * 16 * FS, O_VT = TAB + NFTAB * FTAB;
-  // Derivative terms of mode m at m * DT behind it: d phi_m / d xi_e = c_e phi_(i_e) (+ c_3 phi_0 along the
-  // axis of a pure cubic): D + 1 slots (e * NP + i_e, the cubic's last), their coefficients, and what
-  // rounding took from these.  All modes i are of degree < P, the first NP.
-  static constexpr int NP = tdeg_count(D, P - 1), DT = 3 * (D + 1), O_DT = O_VT + VTAB, SIZE = O_DT + N * DT;
-  static_assert(P <= 3, "one second derivative term per mode");
-  static_assert(VTAB + N * DT <= FTAB, "the JVP kernel keeps the volume table and its terms where the face table goes later");
+  static constexpr int VTAB = TV * 16 * FS, O_VT = O_FT + NFTAB * FTAB, SIZE = O_VT + VTAB;
+  static_assert(VTAB <= FTAB, "the JVP kernel keeps the volume table where the face table goes later");
 };
 
 // Per-axis 1D indices of a node: volume node kv = (i*K1 + j)*K1 + k has x = k, y = j, z = i
@@ -218,7 +220,7 @@ __device__ __forceinline__ void t_test(const Real* tab, const int (&q)[3], int d
 // Copy the first ntab face tables (global memory, after the 1D block) into LDS at ft.
 template <class TS, typename Real>
 __device__ __forceinline__ void ft_load(Real* ft, const Real* gtab, int ntab = 1) {
-  for (int i = threadIdx.x; i < ntab * TS::FTAB; i += blockDim.x) ft[i] = gtab[TS::TAB + i];
+  for (int i = threadIdx.x; i < ntab * TS::FTAB; i += blockDim.x) ft[i] = gtab[TS::O_FT + i];
 }
 
 // Trace contraction from the face trace table: acc[v] (nodes x cells) = FT(face, node, mode) . B.
@@ -269,10 +271,9 @@ __device__ __forceinline__ void t_test_ft(const Real* nrow, const FtCols<TS, Rea
   }
 }
 
-// Volume table and derivative terms.
 template <class TS, typename Real>
 __device__ __forceinline__ void vt_load(Real* vt, const Real* gtab) {
-  for (int i = threadIdx.x; i < TS::VTAB + TS::N * TS::DT; i += blockDim.x) vt[i] = gtab[TS::O_VT + i];
+  for (int i = threadIdx.x; i < TS::VTAB; i += blockDim.x) vt[i] = gtab[TS::O_VT + i];
 }
 
 // Volume test of the Euler forms, sum_e sum_k d_e phi_m g_e, by projection: d_e phi_m is a combination of
@@ -318,9 +319,9 @@ struct QAcc {
   }
 };
 
-// racc[v][m] += sum_e D_e[m][n] Q_e,n through `stage` (16 D NP Real of this wavefront's own); terms: the derivative terms.
+// racc[v][m] += sum_e D_e[m][n] Q_e,n through `stage` (16 D NP Real of this wavefront's own).
 template <class TS, typename Real, int V>
-__device__ __forceinline__ void q_fold(const Real* terms, Real* stage, int col, int grp, const QAcc<TS, Real, V>& q, TAcc<TS, Real, V>& racc) {
+__device__ __forceinline__ void q_fold(const Real* tab, Real* stage, int col, int grp, const QAcc<TS, Real, V>& q, TAcc<TS, Real, V>& racc) {
   typedef QAcc<TS, Real, V> Q;
 #pragma unroll
   for (int v = 0; v < V; v++) {
@@ -341,7 +342,7 @@ __device__ __forceinline__ void q_fold(const Real* terms, Real* stage, int col, 
       }
     __builtin_amdgcn_wave_barrier();
     racc.add(v, grp, [&](int m) {
-      const Real* d = terms + m * TS::DT;
+      const Real* d = tab + TS::O_DT + m * TS::DT;
       constexpr int NT = TS::P == 3 ? TS::D + 1 : TS::D;
       Real s = Real(0), x[NT];
 #pragma unroll
@@ -504,14 +505,14 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
 
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Real* tab = reinterpret_cast<Real*>(smem_raw);
-  for (int i = threadIdx.x; i < TS::TAB; i += blockDim.x) tab[i] = a.tab[i];
+  for (int i = threadIdx.x; i < (PROJ ? TS::O_FT : TS::TAB); i += blockDim.x) tab[i] = a.tab[i];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int cell0 = (SPLIT ? xcd_block(a.nxcd, a.plane_blocks) : xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16;
-  Real* stU = tab + ((TS::TAB + 1) & ~1) + wave * (NARR * 16 * STRIDE);
+  Real* stU = tab + TS::tab_lds(PROJ) + wave * (NARR * 16 * STRIDE);
   Real* stX = stU + 16 * STRIDE;
   // face tables: traces, and the reference-derivative traces where the faces use gradients
-  Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * NARR * 16 * STRIDE;
+  Real* ft = tab + TS::tab_lds(PROJ) + TWAVES * NARR * 16 * STRIDE;
   ft_load<TS>(ft, a.tab, form_face_tables<Form, D>());
   Real* vt = ft + form_face_tables<Form, D>() * TS::FTAB;
   if (PROJ) vt_load<TS>(vt, a.tab);
@@ -602,7 +603,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
     }
   }
 
-  if constexpr (PROJ) q_fold<TS, Real, V>(vt + TS::VTAB, vt + TS::VTAB + N * TS::DT + wave * (16 * D * TS::NP), col, grp, qacc, racc);
+  if constexpr (PROJ) q_fold<TS, Real, V>(tab, vt + TS::VTAB + wave * (16 * D * TS::NP), col, grp, qacc, racc);
 
   // ------------------------------------------------------------------- faces
   const Real pbd = Real(a.fp.penalty_base * a.fp.penalty_deg);
@@ -725,7 +726,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (tensor_min_waves<Real, P>())) kt
   if constexpr (SPLIT) {
     split_put<TS, Real, V>(stU, col, grp, racc);   // own cells' coefficients are not read any more
     __syncthreads();
-    split_sum<Real, NT>(tab + ((TS::TAB + 1) & ~1), NARR * 16 * STRIDE, TAN ? a.out : a.R, cell0, a.J, TAN ? Real(1) : Real(a.alpha),
+    split_sum<Real, NT>(tab + TS::tab_lds(PROJ), NARR * 16 * STRIDE, TAN ? a.out : a.R, cell0, a.J, TAN ? Real(1) : Real(a.alpha),
                         TAN ? Real(0) : Real(a.beta));
     return;
   }
@@ -763,9 +764,9 @@ __global__ void __launch_bounds__(64 * TWAVES, (adjoint_min_waves<Real, P, FUSED
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
   const int cell0 = (xcd_block(a.nxcd, a.plane_blocks) * TWAVES + wave) * 16;
-  Real* stU = tab + ((TS::TAB + 1) & ~1) + wave * (2 * 16 * STRIDE);
+  Real* stU = tab + TS::tab_lds(false) + wave * (2 * 16 * STRIDE);
   Real* stW = stU + 16 * STRIDE;
-  Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * 2 * 16 * STRIDE;   // face tables
+  Real* ft = tab + TS::tab_lds(false) + TWAVES * 2 * 16 * STRIDE;   // face tables
   ft_load<TS>(ft, a.tab, form_face_tables<Form, D>());
   stage16<Real, NT>(stU, STRIDE, a.U, cell0, a.J, lane);
   stage16<Real, NT>(stW, STRIDE, a.X, cell0, a.J, lane);
@@ -1074,13 +1075,14 @@ __global__ void __launch_bounds__(64 * TWAVES, (adjoint_min_waves<Real, P, FUSED
 template <int D, int P, int K1, int V, typename Real>
 constexpr size_t kt_lds_bytes(int narrays) {
   typedef TShape<D, P, K1> TS;
-  return (size_t)(((TS::TAB + 1) & ~1) + TWAVES * narrays * 16 * ((V * TS::N) | 1)) * sizeof(Real);
+  return (size_t)(TS::tab_lds(false) + TWAVES * narrays * 16 * ((V * TS::N) | 1)) * sizeof(Real);
 }
 // kt_forward and kt_adjoint: the same, followed by their face tables
 template <class Form, int D, int P, int K1, typename Real>
 constexpr size_t kt_forward_lds_bytes(int narrays) {
   typedef TShape<D, P, K1> TS;
-  const size_t proj = euler_projects<Form, D, P, Real, false, false>() ? TS::VTAB + TS::N * TS::DT + TWAVES * 16 * D * TS::NP : 0;   // volume table, terms, q_fold staging
+  constexpr bool PROJ = euler_projects<Form, D, P, Real, false, false>();   // terms, volume table, q_fold staging
+  const size_t proj = PROJ ? TS::tab_lds(true) - TS::tab_lds(false) + TS::VTAB + TWAVES * 16 * D * TS::NP : 0;
   return kt_lds_bytes<D, P, K1, Form::V, Real>(narrays) + (form_face_tables<Form, D>() * TS::FTAB + proj) * sizeof(Real);
 }
 
@@ -1118,13 +1120,13 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
 
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Real* tab = reinterpret_cast<Real*>(smem_raw);
-  Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * NSLOT * 64;
+  Real* ft = tab + TS::tab_lds(false) + TWAVES * NSLOT * 64;
   for (int i = threadIdx.x; i < TS::TAB; i += blockDim.x) tab[i] = a.tab[i];
   ft_load<TS>(ft, a.tab);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  Real* buf = tab + ((TS::TAB + 1) & ~1) + wave * (NSLOT * 64);
+  Real* buf = tab + TS::tab_lds(false) + wave * (NSLOT * 64);
   const FtCols<TS, Real, V> ftc(col);
   auto slot = [&](int arr, int v, int r) -> Real& { return buf[((arr * V + v) * 4 + r) * 64 + lane]; };
 
@@ -1348,7 +1350,7 @@ __global__ void __launch_bounds__(64 * TWAVES, (vjp_euler_min_waves<Real, P, FUS
   if constexpr (SPLIT) {
     constexpr int PART = 16 * (NT | 1);
     static_assert(2 * PART <= NSLOT * 64, "both results fit the node buffer");
-    Real* parts = tab + ((TS::TAB + 1) & ~1);
+    Real* parts = tab + TS::tab_lds(false);
     split_put<TS, Real, V>(buf, col, grp, aacc);
     if (FUSED) split_put<TS, Real, V>(buf + PART, col, grp, racc);
     __syncthreads();
@@ -1382,17 +1384,17 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   constexpr int V = Form::V, N = TS::N, NT = V * N, NF = TS::NF, MT = TS::MT;
   constexpr int NSLOT = 3 * V * 4;
 
+  constexpr bool PROJ = euler_projects<Form, D, P, Real, true, SPLIT>();
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Real* tab = reinterpret_cast<Real*>(smem_raw);
-  Real* ft = tab + ((TS::TAB + 1) & ~1) + TWAVES * NSLOT * 64;
-  for (int i = threadIdx.x; i < TS::TAB; i += blockDim.x) tab[i] = a.tab[i];
-  constexpr bool PROJ = euler_projects<Form, D, P, Real, true, SPLIT>();
+  Real* ft = tab + TS::tab_lds(PROJ) + TWAVES * NSLOT * 64;
+  for (int i = threadIdx.x; i < (PROJ ? TS::O_FT : TS::TAB); i += blockDim.x) tab[i] = a.tab[i];
   if (PROJ) vt_load<TS>(ft, a.tab);   // the volume table first; the face table takes its place
   else ft_load<TS>(ft, a.tab);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  Real* buf = tab + ((TS::TAB + 1) & ~1) + wave * (NSLOT * 64);
+  Real* buf = tab + TS::tab_lds(PROJ) + wave * (NSLOT * 64);
   const FtCols<TS, Real, V> ftc(col);
   auto slot = [&](int arr, int v, int r) -> Real& { return buf[((arr * V + v) * 4 + r) * 64 + lane]; };
 
@@ -1506,7 +1508,7 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
   }
 
   if constexpr (PROJ) {
-    q_fold<TS, Real, V>(vt + TS::VTAB, buf, col, grp, qacc, racc);
+    q_fold<TS, Real, V>(tab, buf, col, grp, qacc, racc);
     __syncthreads();
     ft_load<TS>(ft, a.tab);
     __syncthreads();
@@ -1586,7 +1588,7 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
     static_assert(16 * (NT | 1) <= NSLOT * 64, "the result fits the node buffer");
     split_put<TS, Real, V>(buf, col, grp, racc);
     __syncthreads();
-    split_sum<Real, NT>(tab + ((TS::TAB + 1) & ~1), NSLOT * 64, a.out, cell0, a.J, Real(1), Real(0));
+    split_sum<Real, NT>(tab + TS::tab_lds(PROJ), NSLOT * 64, a.out, cell0, a.J, Real(1), Real(0));
     return;
   }
   if (valid) {
@@ -1599,7 +1601,13 @@ __global__ void __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_e
 template <int D, int P, int K1, int V, typename Real>
 constexpr size_t kt_vjp_euler_lds_bytes() {
   typedef TShape<D, P, K1> TS;
-  return (size_t)(((TS::TAB + 1) & ~1) + TWAVES * 3 * V * 4 * 64 + TS::FTAB) * sizeof(Real);
+  return (size_t)(TS::tab_lds(false) + TWAVES * 3 * V * 4 * 64 + TS::FTAB) * sizeof(Real);
+}
+// the JVP's also hold the derivative terms if it projects (its cell-split form does not and is launched with the same)
+template <class Form, int D, int P, int K1, typename Real>
+constexpr size_t kt_jvp_euler_lds_bytes() {
+  typedef TShape<D, P, K1> TS;
+  return (size_t)(TS::tab_lds(euler_projects<Form, D, P, Real, true, false>()) + TWAVES * 3 * Form::V * 4 * 64 + TS::FTAB) * sizeof(Real);
 }
 
 }  // namespace bosss

@@ -21,7 +21,7 @@ struct KernelSet {
   // tensor-table kernels (dg_tensor.hpp): 1D tables in LDS, own coefficients staged in LDS
   int P, ttab_size, t_o_l, t_o_dl, t_o_w, t_o_code, t_k2;
   int t_o_dt, t_o_vt, t_vrows, t_np;   // derivative terms, volume table (offsets, its rows), modes of degree < P
-  int t_o_ft, t_frows, t_fs, t_ftab;   // face tables: offset (after the 1D block), rows per face, row stride, size of one
+  int t_o_ft, t_frows, t_fs, t_ftab;   // face tables: offset (after the derivative terms), rows per face, row stride, size of one
   void (*kt64[NVARIANT])(TArgs<double>);
   void (*kt32[NVARIANT])(TArgs<float>);
   size_t ktlds64[NVARIANT], ktlds32[NVARIANT];
@@ -52,7 +52,8 @@ void set_tensor_linearisations(void (**kt)(TArgs<Real>), size_t* lds) {
     kt[KernelSet::JVP] = kt_jvp_euler<Form, D, P, K1, Real>;
     kt[KernelSet::VJP] = kt_vjp_euler<Form, D, P, K1, Real, false>;
     kt[KernelSet::RES_VJP] = kt_vjp_euler<Form, D, P, K1, Real, true>;
-    lds[KernelSet::JVP] = lds[KernelSet::VJP] = lds[KernelSet::RES_VJP] = kt_vjp_euler_lds_bytes<D, P, K1, Form::V, Real>();
+    lds[KernelSet::JVP] = kt_jvp_euler_lds_bytes<Form, D, P, K1, Real>();
+    lds[KernelSet::VJP] = lds[KernelSet::RES_VJP] = kt_vjp_euler_lds_bytes<D, P, K1, Form::V, Real>();
   } else {
     kt[KernelSet::JVP] = kt_forward<Form, D, P, K1, Real, MODE_JVP>;
     kt[KernelSet::VJP] = kt_adjoint<Form, D, P, K1, Real, false>;
@@ -108,7 +109,7 @@ KernelSet make_kernel_set(int kind) {
   typedef TShape<D, P, K1> TSh;
   k.P = P; k.ttab_size = TSh::SIZE; k.t_o_dt = TSh::O_DT; k.t_o_vt = TSh::O_VT; k.t_vrows = TSh::TV * 16; k.t_np = TSh::NP; k.t_o_l = TSh::O_L; k.t_o_dl = TSh::O_DL; k.t_o_w = TSh::O_W; k.t_o_code = TSh::O_CODE;
   k.t_k2 = TSh::K2;
-  k.t_o_ft = TSh::TAB; k.t_frows = TSh::FROWS; k.t_fs = TSh::FS; k.t_ftab = TSh::FTAB;
+  k.t_o_ft = TSh::O_FT; k.t_frows = TSh::FROWS; k.t_fs = TSh::FS; k.t_ftab = TSh::FTAB;
   k.kt64[KernelSet::RES] = kt_forward<Form, D, P, K1, double, MODE_RES>;
   k.ktlds64[KernelSet::RES] = kt_forward_lds_bytes<Form, D, P, K1, double>(1);
   set_tensor_linearisations<Form, D, P, K1, double>(k.kt64, k.ktlds64);
